@@ -757,7 +757,7 @@ int zfr_multi_create(const zfr_ele_desc_t *descs, const double *const *U, double
           if (descs[i2].order + 1 == N && descs[i2].nDims == cD) agg.nEles += descs[i2].nEles;
         agg.eles_per_block = 0;
         const int defEB = (zk::kMaxThreads / nS) > 0 ? zk::kMaxThreads / nS : 1;
-        const int eb = zk::eles_per_block(&agg, defEB, nops_pad, per_ele, false);
+        const int eb = zk::eles_per_block(&agg, defEB, nops_pad, per_ele, false, false);
         eb_of[shape] = eb;
         const size_t lds = sizeof(double) * (nops_pad + eb * per_ele);
         if (lds > zk::max_lds_n(cD, N)) {

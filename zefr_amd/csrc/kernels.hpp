@@ -1554,25 +1554,49 @@ inline size_t max_lds_n(int D, int N) {
   return nS > kMaxThreads ? kMaxLdsBig : kMaxLds;
 }
 
-// Elements per workgroup: the requested tile, limited by the thread count and the LDS
-// the kernel needs per element (per_ele doubles).
+// The default tile of a launch of its own (EB * nS threads).  The one-sided, divergence and
+// main adjoint kernels (phased) are latency-bound and their phases are separated by
+// barriers, so a workgroup of one wave, whose barriers cost nothing, is their best tile
+// wherever its lanes are well filled; where they are not, and for the launches of one or
+// two phases, the idle lanes cost more than the barriers and the tile of up to four waves
+// with the fewest idle lanes is.  The line, measured on the one-sided kernel and the Euler
+// divergence (one wave against the best-filled tile):
+//   nS = 25, filled to 25/32: viscous 256^2 quads 85 against 74 us, Euler 51 against 46;
+//   nS = 49, filled to 49/64: viscous 192^2 quads 121 against 107, Euler 68 against 60;
+//   nS = 27, filled to 27/32: 40^3 hexes viscous 185 against 194, Euler 113 against 136;
+//   nS = 64: 48^3 hexes viscous 545 against 669 (256 threads), Euler 455 against 557.
+inline int default_tile(int nS, bool phased, long nEles) {
+  const int one = 64 / nS;
+  if (phased && one * nS * 32 >= 64 * 27) return one;
+  int best = one < 1 ? 1 : one, waves = (best * nS + 63) / 64;
+  for (int w = waves + 1; w <= kMaxThreads / 64; w++) {
+    const int eb = 64 * w / nS;
+    if (eb * waves > best * w || (!phased && eb * waves == best * w)) { best = eb; waves = w; }  // more lanes filled
+  }
+  // small meshes: rather >= 1024 workgroups (four per CU) than well filled ones: the
+  // one-wave tile where that leaves as many, else as few elements as do, but never a wave
+  // emptier than it need be (480 quads: of 9 points, 7 per workgroup 7.6 us, one 9.0; of 16
+  // points, 4 per workgroup 6.6 us, one 7.6; of 36 points, one per workgroup 7.3 us, seven 8.0)
+  if (nEles < 1024L * best) {
+    const long eb = (nEles + 1023) / 1024;
+    best = (one >= 1 && (nEles >= 1024L * one || eb < one)) ? one : (int)eb;
+  }
+  return best;
+}
+
+// Elements per workgroup: the requested tile or the default, limited by the thread count
+// and the LDS the kernel needs per element (per_ele doubles).
 // one_wave: the launch's workgroup is EB * nS threads, so that a one-wave tile runs as a
 // one-wave workgroup; false for launches of kMaxThreads-thread workgroups (multi-case
-// launches, persistent plans), where the threads beyond EB * nS would idle
-inline int eles_per_block(const zfr_ele_desc_t *d, int defEB, size_t fixed, size_t per_ele, bool one_wave = true) {
-  int eb = d->eles_per_block > 0 ? d->eles_per_block : defEB;
-  if (d->eles_per_block <= 0) {
-    // small meshes (coarse multigrid levels, small cases): keep >= 1024 workgroups, four
-    // per CU, so that every SIMD holds a wave; the kernels are latency-bound there, and
-    // partly filled waves cost less than idle SIMDs
+// launches, persistent plans), where the threads beyond EB * nS would idle: those fill the
+// 256 threads (defEB elements), or on small meshes keep >= 1024 workgroups.
+inline int eles_per_block(const zfr_ele_desc_t *d, int defEB, size_t fixed, size_t per_ele, bool one_wave,
+                          bool phased) {
+  int eb = d->eles_per_block;
+  if (eb <= 0 && one_wave) eb = default_tile(d->nSpts, phased, d->nEles);
+  else if (eb <= 0) {
     const long per_cu4 = ((long)d->nEles + 1023) / 1024;
-    if (per_cu4 < eb) {
-      eb = per_cu4 < 1 ? 1 : (int)per_cu4;
-      // one-wave workgroups (barriers without cross-wave synchronisation) where they
-      // still leave >= 1024 of them
-      const int eb1 = (64 / d->nSpts) > 0 ? 64 / d->nSpts : 1;
-      if (one_wave && eb1 < eb && ((long)d->nEles + eb1 - 1) / eb1 >= 1024) eb = eb1;
-    }
+    eb = per_cu4 < defEB ? (per_cu4 < 1 ? 1 : (int)per_cu4) : defEB;
   }
   while (eb > 1 && (eb * d->nSpts > kMaxThreads || sizeof(double) * (fixed + eb * per_ele) > kMaxLds)) eb--;
   return eb < 1 ? 1 : eb;
