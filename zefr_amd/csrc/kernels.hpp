@@ -151,29 +151,28 @@ __device__ __forceinline__ int find_case(const long *__restrict__ starts, int nc
 // Flux point f of the reference ordering (src/quads.cpp:86-123, src/hexas.cpp:133-194):
 // normal direction, side (0: the -1 end, 1: the +1 end), first spt of the line through
 // it along 'dim', and that line's spt stride.
+// Selections, no branches: the points of a wave lie on several faces, and a switch makes
+// every wave walk most of its cases one after the other.
 template <int D, int N>
 __device__ __forceinline__ void fpt_info(int f, int &dim, int &side, int &base, int &str) {
   if constexpr (D == 2) {
-    const int face = f / N, j = f - face * N;
-    switch (face) {
-      case 0: dim = 1; side = 0; base = j; break;
-      case 1: dim = 0; side = 1; base = N * j; break;
-      case 2: dim = 1; side = 1; base = N - 1 - j; break;
-      default: dim = 0; side = 0; base = N * (N - 1 - j); break;
-    }
-    str = (dim == 0) ? 1 : N;
+    // faces 0..3: dim 1, 0, 1, 0; side 0, 1, 1, 0; the last two run backwards
+    const int face = f / N, j = f - face * N, odd = face & 1;
+    const int jj = (face >= 2) ? N - 1 - j : j;
+    dim = 1 - odd;
+    side = (face + 1) >> 1 & 1;
+    str = odd ? 1 : N;
+    base = odd ? N * jj : jj;
   } else {
+    // face pairs 0..2 along z, x, y, each - then +; the in-face index k runs backwards on
+    // the + ends of z and x and on the - end of y
     constexpr int NN = N * N;
-    const int face = f / NN, r = f - face * NN, j = r / N, k = r - j * N;
-    switch (face) {
-      case 0: dim = 2; side = 0; base = k + N * j; break;
-      case 1: dim = 2; side = 1; base = (N - 1 - k) + N * j; break;
-      case 2: dim = 0; side = 0; base = N * k + NN * j; break;
-      case 3: dim = 0; side = 1; base = N * (N - 1 - k) + NN * j; break;
-      case 4: dim = 1; side = 0; base = (N - 1 - k) + NN * j; break;
-      default: dim = 1; side = 1; base = k + NN * j; break;
-    }
-    str = (dim == 0) ? 1 : ((dim == 1) ? N : NN);
+    const int face = f / NN, r = f - face * NN, j = r / N, k = r - j * N, pair = face >> 1;
+    side = face & 1;
+    dim = (pair == 0) ? 2 : pair - 1;
+    str = (pair == 0) ? NN : ((pair == 1) ? 1 : N);
+    const int kk = ((pair == 2) ? 1 - side : side) ? N - 1 - k : k;
+    base = ((pair == 1) ? N * kk : kk) + ((pair == 0) ? N * j : NN * j);
   }
 }
 
@@ -239,12 +238,12 @@ __device__ __forceinline__ void stage_U_load(const double *__restrict__ U, const
 #pragma unroll
   for (int k = 0; k < OB; k++) {
     const int i = tid + k * NT;
-    r.ro[k] = (i < S::NOPS) ? a.ops[i] : 0.0;
+    r.ro[k] = a.ops[i < S::NOPS ? i : 0];
   }
 #pragma unroll
   for (int k = 0; k < B; k++) {
     const long i = tid + (long)k * NT;
-    r.ru[k] = (i < n) ? Ub[i] : 0.0;
+    r.ru[k] = Ub[i < n ? i : 0];
   }
 }
 
@@ -292,12 +291,12 @@ __device__ __forceinline__ void stage_U(const double *__restrict__ U, const KArg
 #pragma unroll
   for (int k = 0; k < OB; k++) {
     const int i = tid + k * NT;
-    ro[k] = (i < S::NOPS) ? a.ops[i] : 0.0;
+    ro[k] = a.ops[i < S::NOPS ? i : 0];
   }
 #pragma unroll
   for (int k = 0; k < B; k++) {
     const long i = tid + (long)k * NT;
-    ru[k] = (i < n) ? Ub[i] : 0.0;
+    ru[k] = Ub[i < n ? i : 0];
   }
 #pragma unroll
   for (int k = 0; k < OB; k++) {
