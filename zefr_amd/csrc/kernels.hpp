@@ -678,6 +678,43 @@ __device__ __forceinline__ int owned_fpt(unsigned mask, int k) {
   return 0;  // not reached for k < popcount(mask) * nFF
 }
 
+// A set of faces as a list: the faces in increasing order, four bits each.
+template <int D>
+__device__ __forceinline__ unsigned face_list(unsigned mask) {
+  unsigned list = 0u;
+  int n = 0;
+#pragma unroll
+  for (int b = 0; b < 2 * D; b++) {
+    const unsigned bit = (mask >> b) & 1u;
+    list |= (bit ? (unsigned)b : 0u) << n;
+    n += bit ? 4 : 0;
+  }
+  return list;
+}
+
+// The k-th flux point of a list of faces, its faces taken in order.
+template <int D, int N>
+__device__ __forceinline__ int list_fpt(unsigned list, int k) {
+  using S = Shape<D, N>;
+  const int q = k / S::nFF;
+  return (int)((list >> (4 * q)) & 15u) * S::nFF + (k - q * S::nFF);
+}
+
+// The faces of element e that it owns (bit q = face q): all flux points of a face share its
+// slot, so one partner-map entry per face tells.  Every thread of an element reads the same
+// 2 D entries (a broadcast), which costs one memory round trip and no LDS.
+template <int D, int N>
+__device__ __forceinline__ unsigned owned_faces(const unsigned *__restrict__ nbr, int owner) {
+  using S = Shape<D, N>;
+  unsigned p[2 * D], mask = 0u;
+#pragma unroll
+  for (int q = 0; q < 2 * D; q++) p[q] = nbr[q * S::nFF];
+#pragma unroll
+  for (int q = 0; q < 2 * D; q++)
+    if (nbr_slot<D, N>(p[q]) == owner) mask |= 1u << q;
+  return mask;
+}
+
 // ---------------------------------------------------------------- kernel 1: traces
 // Elements::extrapolate_U (src/elements.cpp:1337-1360): U_fpts = oppE U_spts.  With
 // trace_sel = 1 only the points of faces the partner owns are written: on the one-sided
@@ -1192,7 +1229,7 @@ __global__ __launch_bounds__((Shape<D, N>::kThreads)) void k_divergence_multi(co
 // quad kernels at p = 1..3 spill).
 template <int D, int N, int FC>
 struct OneSidedWaves {
-  static constexpr int value = (D == 3 && N == 4) ? 4 : ((D == 2 && N == 5 && FC == 0) ? 6 : 1);
+  static constexpr int value = (D == 3 && N == 4) ? 4 : ((D == 2 && N == 5 && FC == 0) ? 4 : 1);
 };
 
 // SELF: extrapolate the partner traces this element needs from the partner's U (no trace
@@ -1214,84 +1251,74 @@ __device__ __forceinline__ void visc_onesided_block(const double *__restrict__ U
   double *lops = lds;
   double *lU = lops + S::NOPS_PAD;
   double *lW = lU + EB * V * nS;
-  unsigned *lmask = reinterpret_cast<unsigned *>(lW + EB * W);  // owned faces per element
   const long e0 = bid * EB;
   const long neb = min((long)EB, (long)a.E - e0);
   const int tid = threadIdx.x, el = tid / nS, t = tid - el * nS;
   const long e = e0 + el;
   const bool valid = el < neb;
-  // the slots of this thread's flux points and, where this element owns the face, the
-  // partner's trace: with SELF extrapolated here from the partner's solution line
-  // (no trace launch runs before this kernel), else read from the partner's Utr.  Issued
-  // before the staging barrier so the loads overlap it.
-  // The staging loads and all neighbour entries are issued first, then every partner load,
-  // and only then are values consumed: the prologue costs two dependent memory round trips
-  // rather than two per flux point plus the staging's.
-  int slot[S::FPT];
-  double cp[S::FPT][V];
+  // Work item k of an element is its k-th owned flux point: thread t takes k = t in the
+  // prologue and again in the face phase, so the partner's trace there stays in its
+  // registers (half of the flux points are owned on average, so the items beyond the first
+  // nS are rare for N >= 3; their traces are parked in Utr at this element's own points,
+  // which nothing else reads).  The staging loads are issued first and the partner's values
+  // before any is consumed; with SELF they are its solution line through the point (no
+  // trace launch runs before this kernel), otherwise its trace from Utr.
   constexpr bool self = SELF;
   StageRegs<D, N> sr;
   stage_U_load<D, N>(U, a, e0, neb, sr);
-  unsigned nb[S::FPT];
+  const unsigned mask = valid ? owned_faces<D, N>(a.nbr + e * nF, owner) : 0u;
+  const unsigned owned = face_list<D>(mask), unowned = face_list<D>(~mask);
+  const int cnt = __popc(mask) * S::nFF;
+  double *c = lW + el * W;
+  double cp[V];
+  if (t < cnt && valid) {
+    const int f = list_fpt<D, N>(owned, t);
+    long ep; int sl, fp;
+    unpack_nbr<D, N>(a.nbr[e * nF + f], ep, sl, fp);
+    if constexpr (self) {
+      PartnerLine<D, N> pl;
+      partner_line_load<D, N>(U, a.ops, ep, fp, pl);
+      partner_line_reduce<D, N>(pl, cp);
+    } else {
 #pragma unroll
-  for (int k = 0; k < S::FPT; k++) {
-    const int f = t + k * nS;
-    nb[k] = (valid && f < nF) ? a.nbr[e * nF + f] : 0u;
+      for (int v = 0; v < V; v++) cp[v] = a.Utr[(ep * V + v) * nF + fp];
+    }
+#pragma unroll
+    for (int v = 0; v < V; v++) c[v * nF + f] = cp[v];
   }
-  PartnerLine<D, N> pl[self ? S::FPT : 1];
-  bool own[S::FPT];
+#pragma unroll 1
+  for (int k = t + nS; k < cnt; k += nS) {
+    const int f = list_fpt<D, N>(owned, k);
+    long ep; int sl, fp;
+    unpack_nbr<D, N>(a.nbr[e * nF + f], ep, sl, fp);
+    double x[V];
+    if constexpr (self) {
+      partner_trace<D, N>(U, a.ops, ep, fp, x);
+    } else {
 #pragma unroll
-  for (int k = 0; k < S::FPT; k++) {
-    const int f = t + k * nS;
-    slot[k] = -1;
-    own[k] = false;
-    if (valid && f < nF) {
-      long ep; int sl, fp;
-      unpack_nbr<D, N>(nb[k], ep, sl, fp);
-      slot[k] = sl;
-      own[k] = sl == owner;
-      if (own[k]) {
-        if constexpr (self) {
-          partner_line_load<D, N>(U, a.ops, ep, fp, pl[k]);
-        } else {
+      for (int v = 0; v < V; v++) x[v] = a.Utr[(ep * V + v) * nF + fp];
+    }
 #pragma unroll
-          for (int v = 0; v < V; v++) cp[k][v] = a.Utr[(ep * V + v) * nF + fp];
-        }
-      }
+    for (int v = 0; v < V; v++) {
+      c[v * nF + f] = x[v];
+      a.Utr[(e * V + v) * nF + f] = x[v];
     }
   }
-  if constexpr (self) {
-#pragma unroll
-    for (int k = 0; k < S::FPT; k++)
-      if (own[k]) partner_line_reduce<D, N>(pl[k], cp[k]);
-  }
   stage_U_store<D, N>(U, a, lops, lU, e0, neb, V * nS, sr);
-  if (threadIdx.x < EB) lmask[threadIdx.x] = 0u;
   __syncthreads();
   const double *u = lU + el * V * nS;
-  double *c = lW + el * W;
   double *g_l = lW + el * W;
-  // common solution (= the non-owner side's state) and the mask of owned faces (all flux
-  // points of a face share its slot, so ownership is per face)
+  // common solution (= the non-owner side's state): this element's own trace elsewhere
   if (valid) {
+    const int rest = nF - cnt;
+#pragma unroll 1
+    for (int k = t; k < rest; k += nS) {
+      const int f = list_fpt<D, N>(unowned, k);
+      int dim, side, base, str;
+      fpt_info<D, N>(f, dim, side, base, str);
+      const double *lE = tab_lE<N>(lops, side);
 #pragma unroll
-    for (int k = 0; k < S::FPT; k++) {
-      const int f = t + k * nS;
-      if (f >= nF) continue;
-      if (slot[k] == owner) {
-#pragma unroll
-        for (int v = 0; v < V; v++) {
-          c[v * nF + f] = cp[k][v];
-          if (self) a.Utr[(e * V + v) * nF + f] = cp[k][v];  // own slot: read back in the face phase
-        }
-        if (f % S::nFF == 0) atomicOr(&lmask[el], 1u << (f / S::nFF));
-      } else {
-        int dim, side, base, str;
-        fpt_info<D, N>(f, dim, side, base, str);
-        const double *lE = tab_lE<N>(lops, side);
-#pragma unroll
-        for (int v = 0; v < V; v++) c[v * nF + f] = line_extrap<N>(lE, u + v * nS, base, str);
-      }
+      for (int v = 0; v < V; v++) c[v * nF + f] = line_extrap<N>(lE, u + v * nS, base, str);
     }
   }
   __syncthreads();
@@ -1313,11 +1340,9 @@ __device__ __forceinline__ void visc_onesided_block(const double *__restrict__ U
   __syncthreads();
   // common normal flux (unscaled) at the owned flux points -> Ftr
   if (valid) {
-    const unsigned mask = lmask[el];
-    const int cnt = __popc(mask) * S::nFF;
 #pragma unroll 1
     for (int k = t; k < cnt; k += nS) {
-      const int f = owned_fpt<D, N>(mask, k);  // face-major: neighbouring lanes, neighbouring points
+      const int f = list_fpt<D, N>(owned, k);  // face-major: neighbouring lanes, neighbouring points
       int dim, side, base, str;
       fpt_info<D, N>(f, dim, side, base, str);
       const double *lE = tab_lE<N>(lops, side);
@@ -1328,36 +1353,24 @@ __device__ __forceinline__ void visc_onesided_block(const double *__restrict__ U
       double Uo[V], Up[V];
 #pragma unroll
       for (int v = 0; v < V; v++) Uo[v] = line_extrap<N>(lE, u + v * nS, base, str);
-      if constexpr (FC == 1) {
-        // Roe: the convective flux first, so that its many temporaries are dead before the
-        // gradient's lines are gathered (formed in the Rusanov order it needs ~350 registers)
-        {
-          long ep; int sl, fp;
-          unpack_nbr<D, N>(a.nbr[e * nF + f], ep, sl, fp);
-          const long ip = self ? (e * V * nF + f) : (ep * V * nF + fp);
 #pragma unroll
-          for (int v = 0; v < V; v++) Up[v] = a.Utr[ip + v * nF];
-        }
-        double Fo[V], G[V];
-        if (owner == 0) conv_common_flux<D, FC>(Uo, Up, n, a, Fo);
-        else conv_common_flux<D, FC>(Up, Uo, n, a, Fo);
-        asm volatile("" ::: "memory");
-        visc_normal<D>(Uo, [&](int j, double *dUj) {
+      for (int v = 0; v < V; v++) Up[v] = (k == t) ? cp[v] : a.Utr[(e * V + v) * nF + f];
+      // the convective flux and the LDG penalty first, so that their temporaries and the
+      // partner's state are dead before the gradient's lines are gathered (Roe in the other
+      // order needs ~350 registers)
+      double Fo[V], G[V];
+      if (owner == 0) {
+        conv_common_flux<D, FC>(Uo, Up, n, a, Fo);
 #pragma unroll
-          for (int v = 0; v < V; v++) {
-            dUj[v] = line_extrap<N>(lE, g_l + (j * V + v) * nS, base, str);
-            asm volatile("" : "+v"(dUj[v]) : : "memory");  // formed here, before the next line is loaded
-          }
-        }, n, a, G);
-        if (owner == 0) ldg_common_add<D, BM>(Uo, Up, G, G, a, Fo);
-        else ldg_common_add<D, BM>(Up, Uo, G, G, a, Fo);
+        for (int v = 0; v < V; v++) Fo[v] += a.ldg_tau * (Uo[v] - Up[v]);
+      } else {
+        conv_common_flux<D, FC>(Up, Uo, n, a, Fo);
 #pragma unroll
-        for (int v = 0; v < V; v++) __builtin_nontemporal_store(Fo[v], &a.Ftr[(e * V + v) * nF + f]);
-        continue;
+        for (int v = 0; v < V; v++) Fo[v] += a.ldg_tau * (Up[v] - Uo[v]);
       }
-      double G[V];
-      // one variable's line at a time (a compiler barrier after each): 128 VGPRs instead
-      // of 160, i.e. one more wave per SIMD, worth more than the loads' overlap
+      asm volatile("" ::: "memory");
+      // one variable's line at a time (a compiler barrier after each): 128 VGPRs instead of
+      // 160, i.e. one more wave per SIMD, worth more than the loads' overlap
       visc_normal<D>(Uo, [&](int j, double *dUj) {
 #pragma unroll
         for (int v = 0; v < V; v++) {
@@ -1365,17 +1378,9 @@ __device__ __forceinline__ void visc_onesided_block(const double *__restrict__ U
           asm volatile("" : "+v"(dUj[v]) : : "memory");  // formed here, before the next line is loaded
         }
       }, n, a, G);
-      asm volatile("" ::: "memory");  // load the partner's state only now: fewer live registers
-      {
-        long ep; int sl, fp;
-        unpack_nbr<D, N>(a.nbr[e * nF + f], ep, sl, fp);
-        const long ip = self ? (e * V * nF + f) : (ep * V * nF + fp);  // cached since phase 1
+      // the owner's side alone, with weight 1/2 + |beta| = 1
 #pragma unroll
-        for (int v = 0; v < V; v++) Up[v] = a.Utr[ip + v * nF];
-      }
-      double Fo[V];
-      if (owner == 0) common_flux<D, true, BM, FC>(Uo, Up, G, G, n, 1.0, a, Fo);
-      else common_flux<D, true, BM, FC>(Up, Uo, G, G, n, 1.0, a, Fo);
+      for (int v = 0; v < V; v++) Fo[v] += G[v];
 #pragma unroll
       for (int v = 0; v < V; v++) __builtin_nontemporal_store(Fo[v], &a.Ftr[(e * V + v) * nF + f]);
     }
