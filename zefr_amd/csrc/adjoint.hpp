@@ -76,30 +76,64 @@ __global__ __launch_bounds__((Shape<D, N>::kThreads)) void k_adj_prep(const doub
   }
 }
 
-// LDS per element: U [V][nS]; one region that holds the common solution, then the forward
-// gradient [D][V][nS], then (viscous, once the face adjoint has read the gradient) the own
-// trace cotangent [V][nF]; the gradient cotangent [D][V][nS] (viscous); the own trace
-// cotangent in a region of its own (Euler); the owned-face mask.  w is read from global
-// memory (each value by the few threads of its lines, from cache).  The partner's share
-// of the trace cotangent goes straight to Xtr; __syncthreads orders this block's global
-// accesses too.
+// LDS per element.  Viscous: U [V][nS]; R, which holds the common solution [V][nF], then the
+// forward gradient [D][V][nS], then the gradient-trace cotangents of the owned points
+// [D][V][nS slots], then the own trace cotangent [V][nF]; GB, which holds w [V][nS], then
+// the gradient cotangent [D][V][nS].  Euler: U, w and the own trace cotangent.
 template <int D, int N, bool VISC>
 struct AdjLds {
   using S = Shape<D, N>;
-  static constexpr int R0 = (S::V * S::nF > D * S::V * S::nS) ? S::V * S::nF : D * S::V * S::nS;
-  static constexpr int R = VISC ? R0 : 0;
-  static constexpr int GB = VISC ? D * S::V * S::nS : 0;
-  static constexpr int TO = VISC ? 0 : S::V * S::nF;
-  static constexpr int per_ele = S::V * S::nS + R + GB + TO + 1;  // doubles
+  static constexpr int R = (S::V * S::nF > D * S::V * S::nS || !VISC) ? S::V * S::nF : D * S::V * S::nS;
+  static constexpr int GB = VISC ? D * S::V * S::nS : S::V * S::nS;
+  static constexpr int per_ele = S::V * S::nS + R + GB;  // doubles
 };
 
+// The partner's trace at this thread's owned flux point f: its neighbour entry, then its
+// solution line.
+template <int D, int N>
+__device__ __forceinline__ void owned_partner_trace(const double *__restrict__ U, const KArgs &a, long e, int f,
+                                                    double *out) {
+  long ep; int sl, fp;
+  unpack_nbr<D, N>(a.nbr[e * Shape<D, N>::nF + f], ep, sl, fp);
+  PartnerLine<D, N> pl;
+  partner_line_load<D, N>(U, a.ops, ep, fp, pl);
+  partner_line_reduce<D, N>(pl, out);
+}
+
+// The common flux of one owned point reversed, without its viscous part: Fb = both sides'
+// weights of w, Uo / Up the owner's and the partner's traces.  Adds to Uob (owner's trace)
+// and Gb (the owner's viscous normal flux), writes the partner's share to Upb.
 template <int D, int N, bool VISC, int BM, int FC>
-__device__ __forceinline__ void adj_main_block(const double *__restrict__ U, const double *__restrict__ w,
+__device__ __forceinline__ void owned_flux_vjp(const KArgs &a, const double *__restrict__ Wtr, long e, int f,
+                                               const double *n, const double *Uo, const double *Up, double *Uob,
+                                               double *Upb, double *Gb) {
+  using S = Shape<D, N>;
+  constexpr int nF = S::nF, V = S::V, owner = (BM == 2) ? 1 : 0;
+  long ep; int sl, fp;
+  unpack_nbr<D, N>(a.nbr[e * nF + f], ep, sl, fp);
+  double Fb[V];
+#pragma unroll
+  for (int v = 0; v < V; v++) {
+    Fb[v] = Wtr[(e * V + v) * nF + f] + Wtr[(ep * V + v) * nF + fp];
+    Uob[v] = Upb[v] = Gb[v] = 0.0;
+  }
+  if (owner == 0) common_flux_vjp<D, VISC, BM, FC>(Uo, Up, n, 1.0, a, Fb, Uob, Upb, Gb, nullptr);
+  else common_flux_vjp<D, VISC, BM, FC>(Up, Uo, n, 1.0, a, Fb, Upb, Uob, Gb, nullptr);
+}
+
+// Work item k of an element is its k-th owned flux point (owned faces in increasing
+// order); thread t takes k = t, t + nS, ...: half of the flux points are owned on average,
+// so for N >= 3 one pass covers nearly every element, and thread t's point stays its own
+// from the prologue (its partner's trace) to the end (its own trace's cotangent), in
+// registers.  An element's earlier passes, if it has any, park those values in global
+// memory at the element's own owned points (Utr, Wtr), which no other element reads.
+template <int D, int N, int BM, int FC>
+__device__ __forceinline__ void adj_visc_block(const double *__restrict__ U, const double *__restrict__ w,
                                                double *__restrict__ Wtr, double *__restrict__ Xtr,
                                                double *__restrict__ vout, const KArgs &a, long bid) {
   using S = Shape<D, N>;
-  using L = AdjLds<D, N, VISC>;
-  constexpr int nS = S::nS, nF = S::nF, V = S::V;
+  using L = AdjLds<D, N, true>;
+  constexpr int nS = S::nS, nF = S::nF, V = S::V, nFF = S::nFF;
   constexpr int owner = (BM == 2) ? 1 : 0;
   extern __shared__ double lds[];
   const int EB = a.EB;
@@ -107,123 +141,107 @@ __device__ __forceinline__ void adj_main_block(const double *__restrict__ U, con
   double *lU = lops + S::NOPS_PAD;
   double *lR = lU + EB * V * nS;
   double *lGB = lR + EB * L::R;
-  double *lTo = lGB + EB * L::GB;
-  unsigned *lmask = reinterpret_cast<unsigned *>(lTo + EB * L::TO);  // owned faces per element
   const long e0 = bid * EB;
   const long neb = min((long)EB, (long)a.E - e0);
   const int tid = threadIdx.x, el = tid / nS, t = tid - el * nS;
   const long e = e0 + el;
   const bool valid = el < neb;
-  // the staging loads, this thread's neighbour entries and (viscous) the partner's solution
-  // line at each point this element owns are all issued before any is consumed: two
-  // dependent memory round trips instead of one per flux point after the staging's
+  double *u = lU + el * V * nS;
+  double *c = lR + el * L::R, *g_l = c, *T = c, *to = c;
+  double *gb = lGB + el * L::GB;
+  // 0. staging loads of U and w, the owned faces, and the partner's trace at this thread's
+  //    owned point; only then are values consumed
   StageRegs<D, N> sr;
   stage_U_load<D, N>(U, a, e0, neb, sr);
-  unsigned nb[S::FPT];
+  double wr[V];
 #pragma unroll
-  for (int k = 0; k < S::FPT; k++) {
-    const int f = t + k * nS;
-    nb[k] = (valid && f < nF) ? a.nbr[e * nF + f] : 0u;
+  for (int v = 0; v < V; v++) wr[v] = valid ? w[(e * V + v) * nS + t] : 0.0;
+  const unsigned mask = valid ? owned_faces<D, N>(a.nbr + e * nF, owner) : 0u;
+  const unsigned owned = face_list<D>(mask), unowned = face_list<D>(~mask);
+  const int cnt = __popc(mask) * nFF;
+  // the element's last pass starts at work item 'last' (0 unless more than nS points are owned)
+  const int last = (cnt > nS) ? ((cnt - 1) / nS) * nS : 0;
+  const int klast = t + last;
+  const bool has_last = klast < cnt;
+  double cp[V];
+  if (has_last) {
+    const int f = list_fpt<D, N>(owned, klast);
+    owned_partner_trace<D, N>(U, a, e, f, cp);
+#pragma unroll
+    for (int v = 0; v < V; v++) c[v * nF + f] = cp[v];
   }
-  PartnerLine<D, N> pl[VISC ? S::FPT : 1];
-  double cp[VISC ? S::FPT : 1][V];
-  bool own[S::FPT];
+#pragma unroll 1
+  for (int k = t; k < last; k += nS) {
+    const int f = list_fpt<D, N>(owned, k);
+    double x[V];
+    owned_partner_trace<D, N>(U, a, e, f, x);
 #pragma unroll
-  for (int k = 0; k < S::FPT; k++) {
-    const int f = t + k * nS;
-    own[k] = false;
-    if (valid && f < nF) {
-      long ep; int sl, fp;
-      unpack_nbr<D, N>(nb[k], ep, sl, fp);
-      own[k] = sl == owner;
-      if (VISC && own[k]) partner_line_load<D, N>(U, a.ops, ep, fp, pl[VISC ? k : 0]);
+    for (int v = 0; v < V; v++) {
+      c[v * nF + f] = x[v];
+      a.Utr[(e * V + v) * nF + f] = x[v];
     }
-  }
-  if (VISC) {
-#pragma unroll
-    for (int k = 0; k < S::FPT; k++)
-      if (own[k]) partner_line_reduce<D, N>(pl[VISC ? k : 0], cp[VISC ? k : 0]);
   }
   stage_U_store<D, N>(U, a, lops, lU, e0, neb, V * nS, sr);
-  if (threadIdx.x < EB) lmask[threadIdx.x] = 0u;
-  __syncthreads();
-  const double *u = lU + el * V * nS;
-  const double *we = w + e * V * nS;
-  double *c = lR + el * L::R, *g_l = lR + el * L::R;
-  // viscous: the trace cotangent takes the gradient's region after the face adjoint
-  double *gb = lGB + el * L::GB, *to = VISC ? lR + el * L::R : lTo + el * L::TO;
-  const int ia = t % N, ib = (t / N) % N, ic = (D == 3) ? t / (N * N) : 0;
-  // 1. owned list, zeroed own-trace cotangent, common solution (viscous)
   if (valid) {
 #pragma unroll
-    for (int k = 0; k < S::FPT; k++) {
-      const int f = t + k * nS;
-      if (f >= nF) continue;
-      if (own[k] && f % S::nFF == 0) atomicOr(&lmask[el], 1u << (f / S::nFF));
-      if (VISC) {
-        if (own[k]) {
-          // the partner's trace, from its U; parked in Utr at this element's own point
+    for (int v = 0; v < V; v++) gb[v * nS + t] = wr[v];
+  }
+  __syncthreads();
+  const int ia = t % N, ib = (t / N) % N, ic = (D == 3) ? t / (N * N) : 0;
+  // 1. common solution: this element's own trace where the partner owns the face
+  if (valid) {
+#pragma unroll 1
+    for (int k = t; k < nF - cnt; k += nS) {
+      const int f = list_fpt<D, N>(unowned, k);
+      int dim, side, base, str;
+      fpt_info<D, N>(f, dim, side, base, str);
+      const double *lE = tab_lE<N>(lops, side);
 #pragma unroll
-          for (int v = 0; v < V; v++) {
-            c[v * nF + f] = cp[VISC ? k : 0][v];
-            a.Utr[(e * V + v) * nF + f] = cp[VISC ? k : 0][v];
-          }
-        } else {
-          int dim, side, base, str;
-          fpt_info<D, N>(f, dim, side, base, str);
-          const double *lE = tab_lE<N>(lops, side);
-#pragma unroll
-          for (int v = 0; v < V; v++) c[v * nF + f] = line_extrap<N>(lE, u + v * nS, base, str);
-        }
-      }
-      if (!VISC) {
-#pragma unroll
-        for (int v = 0; v < V; v++) to[v * nF + f] = 0.0;
-      }
+      for (int v = 0; v < V; v++) c[v * nF + f] = line_extrap<N>(lE, u + v * nS, base, str);
     }
   }
   __syncthreads();
-  double ij[D][D], detJ = 1.0;
-  if (valid) load_metric<D>(a, e, t, nS, ij, detJ, VISC);
-  // 2. forward physical gradient at every spt (viscous), into the region of c
-  if (VISC) {
-    double g[V][D];
-    if (valid) spt_gradient<D, N>(lops, u, c, t, ij, detJ, g);
+  // 2. forward physical gradient at every spt, into the region of c; tFb[d1] = Dss^T w along
+  //    the d1 lines
+  double Ub[V], tFb[D][V];
+  {
+    double ij[D][D], detJ, g[V][D];
+    if (valid) {
+      load_metric<D>(a, e, t, nS, ij, detJ, true);
+      spt_gradient<D, N>(lops, u, c, t, ij, detJ, g);
+    }
     __syncthreads();  // the common solution is consumed
     if (valid) {
 #pragma unroll
       for (int d = 0; d < D; d++)
 #pragma unroll
         for (int v = 0; v < V; v++) g_l[(d * V + v) * nS + t] = g[v][d];
+#pragma unroll
+      for (int d = 0; d < D; d++) {
+        const int id = (d == 0) ? ia : ((d == 1) ? ib : ic);
+        const int str = (d == 0) ? 1 : ((d == 1) ? N : N * N);
+#pragma unroll
+        for (int v = 0; v < V; v++) tFb[d][v] = line_T_Dss<N>(lops, id, gb + v * nS, t - id * str, str);
+      }
     }
-    __syncthreads();
-  }
-  // 3. volume adjoint: tFb[d1] = Dss^T w along the d1 lines; F(U, grad) reversed
-  double Ub[V];
+    __syncthreads();  // w is consumed
+    // 3. volume adjoint: F(U, grad) reversed for the cotangent tFb
+    if (valid) {
+      double Us[V];
 #pragma unroll
-  for (int v = 0; v < V; v++) Ub[v] = 0.0;
-  if (valid) {
-    double Us[V];
+      for (int v = 0; v < V; v++) {
+        Us[v] = u[v * nS + t];
+        Ub[v] = 0.0;
+      }
+      const Prim<D> p = primitives<D>(Us, a.gamma);
 #pragma unroll
-    for (int v = 0; v < V; v++) Us[v] = u[v * nS + t];
-    const Prim<D> p = primitives<D>(Us, a.gamma);
-    double tFb[D][V];
-#pragma unroll
-    for (int d = 0; d < D; d++) {
-      const int id = (d == 0) ? ia : ((d == 1) ? ib : ic);
-      const int str = (d == 0) ? 1 : ((d == 1) ? N : N * N);
-      const int base = t - id * str;
-#pragma unroll
-      for (int v = 0; v < V; v++) tFb[d][v] = line_T_Dss<N>(lops, id, we + v * nS, base, str);
-      conv_proj_vjp<D>(Us, p, ij[d], tFb[d], a.gamma, Ub);
-    }
-    if (VISC) {
+      for (int d = 0; d < D; d++) conv_proj_vjp<D>(Us, p, ij[d], tFb[d], a.gamma, Ub);
       // tF[d1] -= T . adj[d1]: cotangent on T[v][j] is -sum_d1 tFb[d1][v] adj[d1][j]
       viscous_vjp<D>(
           Us, p,
           [&](int j, double *dUj) {
 #pragma unroll
-            for (int v = 0; v < V; v++) dUj[v] = g_l[(j * V + v) * nS + t];
+            for (int v = 0; v < V; v++) dUj[v] = g[v][j];
           },
           [&](int v, int j) {
             double s = 0.0;
@@ -238,165 +256,173 @@ __device__ __forceinline__ void adj_main_block(const double *__restrict__ U, con
           a, Ub);
     }
   }
-  __syncthreads();
-  // 4. face adjoint at owned points; the partner's trace cotangent goes to Xtr, the
-  //    gradient cotangent spreads face by face (lines of one face never meet, so the
-  //    accumulation order is fixed)
-  const unsigned mask = valid ? lmask[el] : 0u;
-  const int cnt = __popc(mask) * S::nFF;
-  // viscous: the owned points' trace cotangents go to LDS once the gradient is read; until
-  // then each waits in its own point's Wtr entry, which this thread has just read and no
-  // other element reads (the partner reads Wtr only at the points it owns)
-  int fown[S::FPT];
-#pragma unroll
-  for (int kk = 0; kk < S::FPT; kk++) fown[kk] = -1;
-#pragma unroll
-  for (int kk = 0; kk < S::FPT; kk++) {
-    // viscous runs use one element per workgroup, so cnt is the same for every thread and
-    // a pass with no owned point left (and its barriers) is skipped by all of them
-    if (VISC && kk > 0 && kk * nS >= cnt) break;
-    const int k = t + kk * nS;
-    const bool has = valid && k < cnt;
+  // 4. face adjoint at the owned points.  An owned point's gradient cotangent belongs to the
+  //    spts of its normal line; in the last pass it is left in T, one slot per work item,
+  //    and the spts collect it (phase 5).  T takes the forward gradient's place, so earlier
+  //    passes, which still need that, add to the lines themselves face by face (lines of one
+  //    face never meet, so the order is fixed).
+  double Uob[V];
+#pragma unroll 1
+  for (int k0 = 0; k0 < nF; k0 += nS) {
+    const int k = k0 + t;
+    const bool now = k0 <= last, has = now && k < cnt, fin = k0 == last;
     int f = 0, dim = 0, side = 0, base = 0, str = 0;
     double dGb[V][D];
     if (has) {
-      f = owned_fpt<D, N>(mask, k);
+      f = list_fpt<D, N>(owned, k);
       fpt_info<D, N>(f, dim, side, base, str);
       const double *lE = tab_lE<N>(lops, side);
       const double *fg = a.fgeo + e * (D + 1) * nF + f;
-      double n[D];
-#pragma unroll
-      for (int d = 0; d < D; d++) n[d] = fg[d * nF];
-      double Uo[V], Uob[V], Gb[V];
+      double n[D], Uo[V], Gb[V];
       {
-        long ep; int sl, fp;
-        unpack_nbr<D, N>(a.nbr[e * nF + f], ep, sl, fp);
-        double Up[V], Fb[V], Upb[V];
-        if (VISC) {  // parked in phase 1
+        double Up[V], Upb[V];
 #pragma unroll
-          for (int v = 0; v < V; v++) Up[v] = a.Utr[(e * V + v) * nF + f];
-        } else {
-          partner_trace<D, N>(U, a.ops, ep, fp, Up);
-        }
+        for (int d = 0; d < D; d++) n[d] = fg[d * nF];
 #pragma unroll
         for (int v = 0; v < V; v++) {
           Uo[v] = line_extrap<N>(lE, u + v * nS, base, str);
-          Fb[v] = Wtr[(e * V + v) * nF + f] + Wtr[(ep * V + v) * nF + fp];
-          Uob[v] = Upb[v] = Gb[v] = 0.0;
+          Up[v] = fin ? cp[v] : a.Utr[(e * V + v) * nF + f];
         }
-        if (owner == 0) common_flux_vjp<D, VISC, BM, FC>(Uo, Up, n, 1.0, a, Fb, Uob, Upb, Gb, nullptr);
-        else common_flux_vjp<D, VISC, BM, FC>(Up, Uo, n, 1.0, a, Fb, Upb, Uob, Gb, nullptr);
+        owned_flux_vjp<D, N, true, BM, FC>(a, Wtr, e, f, n, Uo, Up, Uob, Upb, Gb);
 #pragma unroll
         for (int v = 0; v < V; v++) Xtr[(e * V + v) * nF + f] = Upb[v];
       }
       asm volatile("" ::: "memory");
-      if (VISC) {
-        // G = -T(Uo, grad_o) . n
-        const Prim<D> po = primitives<D>(Uo, a.gamma);
-        viscous_vjp<D>(
-            Uo, po,
-            [&](int j, double *dUj) {
+      // G = -T(Uo, grad_o) . n
+      const Prim<D> po = primitives<D>(Uo, a.gamma);
+      viscous_vjp<D>(
+          Uo, po,
+          [&](int j, double *dUj) {
 #pragma unroll
-              for (int v = 0; v < V; v++) {
-                dUj[v] = line_extrap<N>(lE, g_l + (j * V + v) * nS, base, str);
-                asm volatile("" : "+v"(dUj[v]) : : "memory");  // formed here, before the next line is loaded
-              }
-            },
-            [&](int v, int j) { return -Gb[v] * n[j]; },
-            [&](int j, const double *gbj) {
+            for (int v = 0; v < V; v++) {
+              dUj[v] = line_extrap<N>(lE, g_l + (j * V + v) * nS, base, str);
+              asm volatile("" : "+v"(dUj[v]) : : "memory");  // formed here, before the next line is loaded
+            }
+          },
+          [&](int v, int j) { return -Gb[v] * n[j]; },
+          [&](int j, const double *gbj) {
 #pragma unroll
-              for (int v = 0; v < V; v++) dGb[v][j] = gbj[v];
-            },
-            a, Uob);
-      }
-      if (VISC) {
-        fown[kk] = f;
-#pragma unroll
-        for (int v = 0; v < V; v++) Wtr[(e * V + v) * nF + f] = Uob[v];
-      } else {
-#pragma unroll
-        for (int v = 0; v < V; v++) to[v * nF + f] = Uob[v];
-      }
+            for (int v = 0; v < V; v++) dGb[v][j] = gbj[v];
+          },
+          a, Uob);
     }
-    if (VISC) {
-      const int face = has ? f / S::nFF : -1;
-      const double *lE = tab_lE<N>(lops, side);
+    // a pass that is not the last of some element (the same for every thread)
+    const bool more = __syncthreads_or(k0 < last);
+    if (now && fin && has) {  // the forward gradient of this element is consumed
+#pragma unroll
+      for (int j = 0; j < D; j++)
+#pragma unroll
+        for (int v = 0; v < V; v++) T[(j * V + v) * nS + t] = dGb[v][j];
+    }
+    if (!more) break;
+    const int face = (has && !fin) ? f / nFF : -1;
+    if (face >= 0) {
+#pragma unroll
+      for (int v = 0; v < V; v++) Wtr[(e * V + v) * nF + f] = Uob[v];
+    }
 #pragma unroll 1
-      for (int q = 0; q < 2 * D; q++) {
-        __syncthreads();
-        if (face == q) {
+    for (int q = 0; q < 2 * D; q++) {
+      __syncthreads();
+      if (face == q) {
+        const double *lE = tab_lE<N>(lops, side);
+#pragma unroll 1
+        for (int m = 0; m < N; m++)
 #pragma unroll
-          for (int m = 0; m < N; m++)
+          for (int j = 0; j < D; j++)
 #pragma unroll
-            for (int j = 0; j < D; j++)
-#pragma unroll
-              for (int v = 0; v < V; v++) gb[(j * V + v) * nS + base + m * str] += lE[m] * dGb[v][j];
-        }
+            for (int v = 0; v < V; v++) gb[(j * V + v) * nS + base + m * str] += lE[m] * dGb[v][j];
       }
     }
   }
   __syncthreads();
-  if (VISC) {
-    // the forward gradient is consumed: its region takes the trace cotangent, owned points
-    // from the face adjoint, the others in phase 6
+  // 5. each spt collects the gradient-trace cotangents of the owned ends of its lines, then
+  //    reference-space gradient cotangent: grb[d2][v] = sum_d1 adj[d2][d1] gb[v][d1] / detJ
+  //    (the metric read again here: held across the face adjoint it takes registers the
+  //    Roe reverse sweep needs)
+  if (valid) {
+    asm volatile("" ::: "memory");
+    double ij[D][D], detJ;
+    load_metric<D>(a, e, t, nS, ij, detJ, true);
+    double gv[V][D];
 #pragma unroll
-    for (int kk = 0; kk < S::FPT; kk++) {
-      if (fown[kk] < 0) continue;
+    for (int j = 0; j < D; j++)
 #pragma unroll
-      for (int v = 0; v < V; v++) to[v * nF + fown[kk]] = Wtr[(e * V + v) * nF + fown[kk]];
-    }
-    // 5. reference-space gradient cotangent: grb[d2][v] = sum_d1 adj[d2][d1] gb[v][d1] / detJ
-    //    (the metric read again here: held across the face adjoint it takes registers the
-    //    Roe reverse sweep needs)
-    if (valid) {
-      asm volatile("" ::: "memory");
-      load_metric<D>(a, e, t, nS, ij, detJ, true);
-      double gv[V][D];
+      for (int v = 0; v < V; v++) gv[v][j] = gb[(j * V + v) * nS + t];
 #pragma unroll
-      for (int j = 0; j < D; j++)
+    for (int d = 0; d < D; d++) {
+      const int id = (d == 0) ? ia : ((d == 1) ? ib : ic);
 #pragma unroll
-        for (int v = 0; v < V; v++) gv[v][j] = gb[(j * V + v) * nS + t];
-      const double inv_det = 1.0 / detJ;
+      for (int sd = 0; sd < 2; sd++) {
+        const int f = fpt_end<D, N>(ia, ib, ic, d, sd);
+        const int q = f / nFF;  // the same face for every spt: its end of direction d
+        const int k = __popc(mask & ((1u << q) - 1u)) * nFF + (f - q * nFF);
+        if (((mask >> q) & 1u) && k >= last) {
+          const double l = tab_lE<N>(lops, sd)[id];
+          const double *Tk = T + (k - last);
 #pragma unroll
-      for (int d2 = 0; d2 < D; d2++)
+          for (int j = 0; j < D; j++)
 #pragma unroll
-        for (int v = 0; v < V; v++) {
-          double s = 0.0;
-#pragma unroll
-          for (int d1 = 0; d1 < D; d1++) s += ij[d2][d1] * gv[v][d1];
-          gb[(d2 * V + v) * nS + t] = s * inv_det;
-        }
-    }
-    __syncthreads();
-    // 6. Dss^T into U, Dsf^T into the common solution's cotangent: the partner's trace at
-    //    owned points (Xtr), this element's trace elsewhere
-    if (valid) {
-#pragma unroll
-      for (int d = 0; d < D; d++) {
-        const int id = (d == 0) ? ia : ((d == 1) ? ib : ic);
-        const int str = (d == 0) ? 1 : ((d == 1) ? N : N * N);
-        const int base = t - id * str;
-#pragma unroll
-        for (int v = 0; v < V; v++) Ub[v] += line_T_Dss<N>(lops, id, gb + (d * V + v) * nS, base, str);
-      }
-#pragma unroll
-      for (int k = 0; k < S::FPT; k++) {
-        const int f = t + k * nS;
-        if (f >= nF) continue;
-        int dim, side, base, str;
-        fpt_info<D, N>(f, dim, side, base, str);
-        long ep; int sl, fp;
-        unpack_nbr<D, N>(a.nbr[e * nF + f], ep, sl, fp);
-#pragma unroll
-        for (int v = 0; v < V; v++) {
-          const double cb = line_Dsf<N>(lops, side, gb + (dim * V + v) * nS, base, str);
-          if (sl == owner) Xtr[(e * V + v) * nF + f] += cb;
-          else to[v * nF + f] = cb;  // this point's only contribution (the face adjoint wrote owned ones)
+            for (int v = 0; v < V; v++) gv[v][j] += l * Tk[(j * V + v) * nS];
         }
       }
     }
-    __syncthreads();
+    const double inv_det = 1.0 / detJ;
+#pragma unroll
+    for (int d2 = 0; d2 < D; d2++)
+#pragma unroll
+      for (int v = 0; v < V; v++) {
+        double s = 0.0;
+#pragma unroll
+        for (int d1 = 0; d1 < D; d1++) s += ij[d2][d1] * gv[v][d1];
+        gb[(d2 * V + v) * nS + t] = s * inv_det;
+      }
   }
+  __syncthreads();
+  // 6. Dss^T into U, Dsf^T into the common solution's cotangent: the partner's trace at
+  //    owned points (Xtr), this element's trace elsewhere
+  if (valid) {
+#pragma unroll
+    for (int d = 0; d < D; d++) {
+      const int id = (d == 0) ? ia : ((d == 1) ? ib : ic);
+      const int str = (d == 0) ? 1 : ((d == 1) ? N : N * N);
+#pragma unroll
+      for (int v = 0; v < V; v++) Ub[v] += line_T_Dss<N>(lops, id, gb + (d * V + v) * nS, t - id * str, str);
+    }
+    auto dsf = [&](int f, double *cb) {
+      int dim, side, base, str;
+      fpt_info<D, N>(f, dim, side, base, str);
+#pragma unroll
+      for (int v = 0; v < V; v++) cb[v] = line_Dsf<N>(lops, side, gb + (dim * V + v) * nS, base, str);
+    };
+    double cb[V];
+    if (has_last) {
+      const int f = list_fpt<D, N>(owned, klast);
+      dsf(f, cb);
+#pragma unroll
+      for (int v = 0; v < V; v++) {
+        Xtr[(e * V + v) * nF + f] += cb[v];
+        to[v * nF + f] = Uob[v];
+      }
+    }
+#pragma unroll 1
+    for (int k = t; k < last; k += nS) {
+      const int f = list_fpt<D, N>(owned, k);
+      dsf(f, cb);
+#pragma unroll
+      for (int v = 0; v < V; v++) {
+        Xtr[(e * V + v) * nF + f] += cb[v];
+        to[v * nF + f] = Wtr[(e * V + v) * nF + f];
+      }
+    }
+#pragma unroll 1
+    for (int k = t; k < nF - cnt; k += nS) {
+      const int f = list_fpt<D, N>(unowned, k);
+      dsf(f, cb);
+#pragma unroll
+      for (int v = 0; v < V; v++) to[v * nF + f] = cb[v];
+    }
+  }
+  __syncthreads();
   if (!valid) return;
   // 7. own trace cotangent E^T into v
 #pragma unroll
@@ -411,8 +437,125 @@ __device__ __forceinline__ void adj_main_block(const double *__restrict__ U, con
   for (int v = 0; v < V; v++) vout[(e * V + v) * nS + t] = Ub[v];
 }
 
+// Euler: the volume adjoint, the face adjoint at the owned points (slot 0), and E^T.
+template <int D, int N, int FC>
+__device__ __forceinline__ void adj_euler_block(const double *__restrict__ U, const double *__restrict__ w,
+                                                const double *__restrict__ Wtr, double *__restrict__ Xtr,
+                                                double *__restrict__ vout, const KArgs &a, long bid) {
+  using S = Shape<D, N>;
+  using L = AdjLds<D, N, false>;
+  constexpr int nS = S::nS, nF = S::nF, V = S::V;
+  extern __shared__ double lds[];
+  const int EB = a.EB;
+  double *lops = lds;
+  double *lU = lops + S::NOPS_PAD;
+  double *lT = lU + EB * V * nS;
+  double *lw = lT + EB * L::R;
+  const long e0 = bid * EB;
+  const long neb = min((long)EB, (long)a.E - e0);
+  const int tid = threadIdx.x, el = tid / nS, t = tid - el * nS;
+  const long e = e0 + el;
+  const bool valid = el < neb;
+  StageRegs<D, N> sr;
+  stage_U_load<D, N>(U, a, e0, neb, sr);
+  double wr[V];
+#pragma unroll
+  for (int v = 0; v < V; v++) wr[v] = valid ? w[(e * V + v) * nS + t] : 0.0;
+  const unsigned mask = valid ? owned_faces<D, N>(a.nbr + e * nF, 0) : 0u;
+  const unsigned owned = face_list<D>(mask);
+  const int cnt = __popc(mask) * S::nFF;
+  double ij[D][D], detJ;
+  if (valid) load_metric<D>(a, e, t, nS, ij, detJ, false);
+  double cp[V];
+  if (t < cnt) owned_partner_trace<D, N>(U, a, e, list_fpt<D, N>(owned, t), cp);
+  stage_U_store<D, N>(U, a, lops, lU, e0, neb, V * nS, sr);
+  const double *u = lU + el * V * nS;
+  double *to = lT + el * L::R, *we = lw + el * V * nS;
+  if (valid) {
+#pragma unroll
+    for (int v = 0; v < V; v++) we[v * nS + t] = wr[v];
+    for (int k = t; k < V * nF; k += nS) to[k] = 0.0;
+  }
+  __syncthreads();
+  const int ia = t % N, ib = (t / N) % N, ic = (D == 3) ? t / (N * N) : 0;
+  double Ub[V];
+  if (valid) {
+#pragma unroll 1
+    for (int k = t; k < cnt; k += nS) {
+      const int f = list_fpt<D, N>(owned, k);
+      int dim, side, base, str;
+      fpt_info<D, N>(f, dim, side, base, str);
+      const double *lE = tab_lE<N>(lops, side);
+      const double *fg = a.fgeo + e * (D + 1) * nF + f;
+      double n[D], Uo[V], Up[V], Uob[V], Upb[V], Gb[V];
+#pragma unroll
+      for (int d = 0; d < D; d++) n[d] = fg[d * nF];
+      if (k == t) {
+#pragma unroll
+        for (int v = 0; v < V; v++) Up[v] = cp[v];
+      } else {
+        owned_partner_trace<D, N>(U, a, e, f, Up);
+      }
+#pragma unroll
+      for (int v = 0; v < V; v++) Uo[v] = line_extrap<N>(lE, u + v * nS, base, str);
+      owned_flux_vjp<D, N, false, 0, FC>(a, Wtr, e, f, n, Uo, Up, Uob, Upb, Gb);
+#pragma unroll
+      for (int v = 0; v < V; v++) {
+        Xtr[(e * V + v) * nF + f] = Upb[v];
+        to[v * nF + f] = Uob[v];
+      }
+    }
+    // volume adjoint: Dss^T w along the lines, the flux reversed
+    double Us[V];
+#pragma unroll
+    for (int v = 0; v < V; v++) {
+      Us[v] = u[v * nS + t];
+      Ub[v] = 0.0;
+    }
+    const Prim<D> p = primitives<D>(Us, a.gamma);
+#pragma unroll
+    for (int d = 0; d < D; d++) {
+      const int id = (d == 0) ? ia : ((d == 1) ? ib : ic);
+      const int str = (d == 0) ? 1 : ((d == 1) ? N : N * N);
+      double tFb[V];
+#pragma unroll
+      for (int v = 0; v < V; v++) tFb[v] = line_T_Dss<N>(lops, id, we + v * nS, t - id * str, str);
+      conv_proj_vjp<D>(Us, p, ij[d], tFb, a.gamma, Ub);
+    }
+  }
+  __syncthreads();
+  if (!valid) return;
+#pragma unroll
+  for (int d = 0; d < D; d++) {
+    const int id = (d == 0) ? ia : ((d == 1) ? ib : ic);
+    const double l0 = tab_lE<N>(lops, 0)[id], l1 = tab_lE<N>(lops, 1)[id];
+    const int f0 = fpt_end<D, N>(ia, ib, ic, d, 0), f1 = fpt_end<D, N>(ia, ib, ic, d, 1);
+#pragma unroll
+    for (int v = 0; v < V; v++) Ub[v] += l0 * to[v * nF + f0] + l1 * to[v * nF + f1];
+  }
+#pragma unroll
+  for (int v = 0; v < V; v++) vout[(e * V + v) * nS + t] = Ub[v];
+}
+
 template <int D, int N, bool VISC, int BM, int FC>
-__global__ __launch_bounds__((Shape<D, N>::kThreads)) __attribute__((amdgpu_waves_per_eu(2)))
+__device__ __forceinline__ void adj_main_block(const double *__restrict__ U, const double *__restrict__ w,
+                                               double *__restrict__ Wtr, double *__restrict__ Xtr,
+                                               double *__restrict__ vout, const KArgs &a, long bid) {
+  if constexpr (VISC) adj_visc_block<D, N, BM, FC>(U, w, Wtr, Xtr, vout, a, bid);
+  else adj_euler_block<D, N, FC>(U, w, Wtr, Xtr, vout, a, bid);
+}
+
+// Occupancy target of the main adjoint kernels: three waves per SIMD (168 VGPRs) where they
+// fit it with at most a few spills, else two (256 VGPRs): held to three, 26^3 hexes p = 2
+// Euler with Roe took 129 us instead of 80 (58 spills), 100^2 quads p = 2 with Rusanov + LDG
+// 29 us instead of 25 (42 spills), while 20^2 x 27 hexes p = 3 Euler went from 80 to 76.
+template <int D, int N, bool VISC, int FC>
+struct AdjWaves {
+  static constexpr int value = FC == 0 && (!VISC || (D == 2 && (N == 4 || N == 5))) ? 3 : 2;
+};
+
+template <int D, int N, bool VISC, int BM, int FC>
+__global__ __launch_bounds__((Shape<D, N>::kThreads)) __attribute__((amdgpu_waves_per_eu(AdjWaves<D, N, VISC, FC>::value)))
 void k_adj_main(const double *__restrict__ U, const double *__restrict__ w, double *__restrict__ Wtr,
                 double *__restrict__ Xtr, double *__restrict__ vout, KArgs a) {
   adj_main_block<D, N, VISC, BM, FC>(U, w, Wtr, Xtr, vout, a, xcd_block(blockIdx.x, gridDim.x));
@@ -421,7 +564,7 @@ void k_adj_main(const double *__restrict__ U, const double *__restrict__ w, doub
 // The same kernel for workgroups of one wave (the viscous adjoint runs one element per
 // workgroup; one wave for hex p=3): its barriers need no cross-wave synchronisation.
 template <int D, int N, bool VISC, int BM, int FC>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2)))
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(AdjWaves<D, N, VISC, FC>::value)))
 void k_adj_main_w64(const double *__restrict__ U, const double *__restrict__ w, double *__restrict__ Wtr,
                     double *__restrict__ Xtr, double *__restrict__ vout, KArgs a) {
   adj_main_block<D, N, VISC, BM, FC>(U, w, Wtr, Xtr, vout, a, xcd_block(blockIdx.x, gridDim.x));
@@ -484,8 +627,8 @@ __global__ __launch_bounds__((Shape<D, N>::kThreads)) void k_adj_gather(const do
 //   k_adj_face     : per flux-point pair, by its slot-0 side: the common flux reversed for
 //                    both sides' states and gradient traces; the cotangents overwrite the
 //                    traces in place (Utr -> d/dUtr, Gtr -> d/dGtr);
-//   k_adj_main_gen : per element: volume adjoint, the gradient-trace cotangents spread
-//                    back along the normal lines, the gradient reversed into U and into the
+//   k_adj_main_gen : per element: volume adjoint, the gradient-trace cotangents collected
+//                    along the normal lines, the gradient reversed into U and into the
 //                    common solution, whose cotangent splits (1/2 -+ beta) between this
 //                    element's trace (with the face part, E^T into v) and the partner's
 //                    (Xtr, at every point);

@@ -662,22 +662,6 @@ __device__ __forceinline__ void pmg_epilogue(const KArgs &a, double *lops, const
   }
 }
 
-// The k-th owned flux point, owned faces taken in increasing order (mask bit q = face q).
-template <int D, int N>
-__device__ __forceinline__ int owned_fpt(unsigned mask, int k) {
-  using S = Shape<D, N>;
-  int q = k / S::nFF;
-  const int r = k - q * S::nFF;
-#pragma unroll
-  for (int b = 0; b < 2 * D; b++) {
-    if ((mask >> b) & 1u) {
-      if (q == 0) return b * S::nFF + r;
-      q--;
-    }
-  }
-  return 0;  // not reached for k < popcount(mask) * nFF
-}
-
 // A set of faces as a list: the faces in increasing order, four bits each.
 template <int D>
 __device__ __forceinline__ unsigned face_list(unsigned mask) {

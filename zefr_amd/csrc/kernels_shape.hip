@@ -34,7 +34,9 @@ void launch_div(const zfr_ele_desc_t *d, dim3 grid, dim3 block, size_t lds, hipS
 template <int D, int N, int FC>
 void launch_adj_main(const zfr_ele_desc_t *d, dim3 grid, dim3 block, size_t lds, hipStream_t st, const double *U,
                      const AdjPtrs &j, double *out, const KArgs &a) {
-  if (!d->viscous)
+  if (!d->viscous && block.x <= 64)
+    hipLaunchKernelGGL((k_adj_main_w64<D, N, false, 0, FC>), grid, block, lds, st, U, j.w, j.Wtr, j.Xtr, out, a);
+  else if (!d->viscous)
     hipLaunchKernelGGL((k_adj_main<D, N, false, 0, FC>), grid, block, lds, st, U, j.w, j.Wtr, j.Xtr, out, a);
   else if (block.x <= 64) {
     if (d->ldg_b == 0.5)
@@ -71,13 +73,9 @@ int launch(Op op, const zfr_ele_desc_t *d, const double *U, double *out, hipStre
   if ((op == Op::OneSided || op == Op::OneSidedFromTrace || op == Op::FaceCorr) && d->ldg_b != 0.5 &&
       d->ldg_b != -0.5)
     return zfr::fail("one-sided LDG kernels need ldg_b = +-0.5");
-  // the viscous adjoint runs one element per workgroup: its LDS then allows ~7
-  // workgroups per CU, more than any larger tile
   const bool phased = op == Op::OneSided || op == Op::OneSidedFromTrace || op == Op::Div || op == Op::AdjMain ||
                       op == Op::AdjMainGen;
-  const int EB = (op == Op::AdjMain && d->viscous)
-                     ? 1
-                     : eles_per_block(d, S::defaultEB(), S::NOPS_PAD, per_ele, !g_persist, phased);
+  const int EB = eles_per_block(d, S::defaultEB(), S::NOPS_PAD, per_ele, !g_persist, phased);
   if (sizeof(double) * (S::NOPS_PAD + EB * per_ele) > max_lds<D, N>())
     return zfr::fail("kernel launch: one element needs more LDS than a workgroup may use (order too high)");
   KArgs a = make_args(d, EB);

@@ -650,16 +650,19 @@ ZFR_HD void common_flux_vjp(const double *UL, const double *UR, const double *n,
     Fs[v] = Fb[v] * dAs;
     Fh[v] = 0.5 * Fs[v];
   }
-  conv_proj_vjp<D>(UL, pL, n, Fh, a.gamma, ULb);
-  conv_proj_vjp<D>(UR, pR, n, Fh, a.gamma, URb);
   if (FC == 1) {
+    // the dissipation first: its many temporaries are dead before the other parts are added
     double db[V];
     ZFR_UNROLL
     for (int v = 0; v < V; v++) db[v] = -Fh[v];
     roe_dissipation_vjp<D>(UL, UR, pL, pR, n, a.gamma, db, ULb, URb);
+    conv_proj_vjp<D>(UL, pL, n, Fh, a.gamma, ULb);
+    conv_proj_vjp<D>(UR, pR, n, Fh, a.gamma, URb);
     if (VISC) ldg_vjp_add<D, BM>(Fs, a, ULb, URb, G1b, G2b);
     return;
   }
+  conv_proj_vjp<D>(UL, pL, n, Fh, a.gamma, ULb);
+  conv_proj_vjp<D>(UR, pR, n, Fh, a.gamma, URb);
   double mnL = UL[1] * n[0], mnR = UR[1] * n[0];
   ZFR_UNROLL
   for (int d = 1; d < D; d++) {
@@ -678,9 +681,34 @@ ZFR_HD void common_flux_vjp(const double *UL, const double *UR, const double *n,
     dissb -= Fs[v] * (UR[v] - UL[v]);
   }
   const double eigb = 0.5 * (1.0 - a.rus_k) * dissb;
-  if (lamL >= lamR) wavespeed_vjp<D>(UL, pL, n, a.gamma, eigb, ULb);
-  else wavespeed_vjp<D>(UR, pR, n, a.gamma, eigb, URb);
-  if (VISC) ldg_vjp_add<D, BM>(Fs, a, ULb, URb, G1b, G2b);
+  if (VISC) {
+    if (lamL >= lamR) wavespeed_vjp<D>(UL, pL, n, a.gamma, eigb, ULb);
+    else wavespeed_vjp<D>(UR, pR, n, a.gamma, eigb, URb);
+    ldg_vjp_add<D, BM>(Fs, a, ULb, URb, G1b, G2b);
+    return;
+  }
+  // inviscid: the side that set the maximum is selected by value, so that no pointer is chosen
+  // at run time (the two branches merge into one, with the cotangents in scratch memory;
+  // the viscous kernels, where they do not, have no registers for the selected copies)
+  const bool left = lamL >= lamR;
+  double Us[V], Ub[V];
+  Prim<D> ps;
+  ps.invrho = left ? pL.invrho : pR.invrho;
+  ps.P = left ? pL.P : pR.P;
+  ps.H = 0.0;
+  ZFR_UNROLL
+  for (int d = 0; d < D; d++) ps.vel[d] = left ? pL.vel[d] : pR.vel[d];
+  ZFR_UNROLL
+  for (int v = 0; v < V; v++) {
+    Us[v] = left ? UL[v] : UR[v];
+    Ub[v] = 0.0;
+  }
+  wavespeed_vjp<D>(Us, ps, n, a.gamma, eigb, Ub);
+  ZFR_UNROLL
+  for (int v = 0; v < V; v++) {
+    ULb[v] += left ? Ub[v] : 0.0;
+    URb[v] += left ? 0.0 : Ub[v];
+  }
 }
 
 }  // namespace zphys
