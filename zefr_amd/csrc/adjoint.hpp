@@ -706,12 +706,13 @@ __global__ __launch_bounds__(kMaxThreads) void k_adj_face(const double *__restri
     }
 }
 
-// LDS per element: U [V][nS]; one region for the common solution, then the forward
-// gradient [D][V][nS], then the trace cotangent [V][nF]; the gradient cotangent [D][V][nS].
+// LDS per element: U [V][nS]; R, which holds the common solution [V][nF], then one
+// direction's gradient-trace cotangents [D][V][2 nFF] at a time, then the trace cotangent
+// [V][nF]; GB, which holds w [V][nS], then the gradient cotangent [D][V][nS].
 template <int D, int N>
 struct AdjGenLds {
   using S = Shape<D, N>;
-  static constexpr int R = (S::V * S::nF > D * S::V * S::nS) ? S::V * S::nF : D * S::V * S::nS;
+  static constexpr int R = (2 * D * S::V * S::nFF > S::V * S::nF) ? 2 * D * S::V * S::nFF : S::V * S::nF;
   static constexpr int per_ele = S::V * S::nS + R + D * S::V * S::nS;  // doubles
 };
 
@@ -721,7 +722,7 @@ __device__ __forceinline__ void adj_main_general_block(const double *__restrict_
                                                        const KArgs &a, long bid) {
   using S = Shape<D, N>;
   using L = AdjGenLds<D, N>;
-  constexpr int nS = S::nS, nF = S::nF, V = S::V;
+  constexpr int nS = S::nS, nF = S::nF, V = S::V, nFF = S::nFF;
   extern __shared__ double lds[];
   const int EB = a.EB;
   double *lops = lds;
@@ -730,15 +731,20 @@ __device__ __forceinline__ void adj_main_general_block(const double *__restrict_
   double *lGB = lR + EB * L::R;
   const long e0 = bid * EB;
   const long neb = min((long)EB, (long)a.E - e0);
-  stage_U<D, N>(U, a, lops, lU, e0, neb, V * nS);
-  __syncthreads();
   const int tid = threadIdx.x, el = tid / nS, t = tid - el * nS;
   const long e = e0 + el;
   const bool valid = el < neb;
   const double *u = lU + el * V * nS;
-  const double *we = w + e * V * nS;
-  double *c = lR + el * L::R, *g_l = c, *to = c;
+  double *c = lR + el * L::R, *T = c, *to = c;
   double *gb = lGB + el * D * V * nS;
+  StageRegs<D, N> sr;
+  stage_U_load<D, N>(U, a, e0, neb, sr);
+  if (valid) {
+#pragma unroll
+    for (int v = 0; v < V; v++) gb[v * nS + t] = w[(e * V + v) * nS + t];
+  }
+  stage_U_store<D, N>(U, a, lops, lU, e0, neb, V * nS, sr);
+  __syncthreads();
   const int ia = t % N, ib = (t / N) % N, ic = (D == 3) ? t / (N * N) : 0;
   const double beta = a.ldg_b;
   // 1. common solution, the partner's trace extrapolated from its U (Utr now holds cotangents)
@@ -763,99 +769,104 @@ __device__ __forceinline__ void adj_main_general_block(const double *__restrict_
     }
   }
   __syncthreads();
-  double ij[D][D], detJ = 1.0;
-  if (valid) load_metric<D>(a, e, t, nS, ij, detJ, true);
-  // 2. forward physical gradient, into the common solution's region
-  {
-    double g[V][D];
-    if (valid) spt_gradient<D, N>(lops, u, c, t, ij, detJ, g);
-    __syncthreads();
-    if (valid) {
-#pragma unroll
-      for (int d = 0; d < D; d++)
-#pragma unroll
-        for (int v = 0; v < V; v++) g_l[(d * V + v) * nS + t] = g[v][d];
-    }
-    __syncthreads();
-  }
-  // 3. volume adjoint: tFb[d1] = Dss^T w along the d1 lines; F(U, grad) reversed
+  // 2. forward physical gradient at this thread's spt; tFb[d1] = Dss^T w along the d1 lines
   double Ub[V];
+  {
+    double ij[D][D], detJ, g[V][D], tFb[D][V];
+    if (valid) {
+      load_metric<D>(a, e, t, nS, ij, detJ, true);
+      spt_gradient<D, N>(lops, u, c, t, ij, detJ, g);
 #pragma unroll
-  for (int v = 0; v < V; v++) Ub[v] = 0.0;
-  if (valid) {
-    double Us[V];
+      for (int d = 0; d < D; d++) {
+        const int id = (d == 0) ? ia : ((d == 1) ? ib : ic);
+        const int str = (d == 0) ? 1 : ((d == 1) ? N : N * N);
 #pragma unroll
-    for (int v = 0; v < V; v++) Us[v] = u[v * nS + t];
-    const Prim<D> p = primitives<D>(Us, a.gamma);
-    double tFb[D][V];
-#pragma unroll
-    for (int d = 0; d < D; d++) {
-      const int id = (d == 0) ? ia : ((d == 1) ? ib : ic);
-      const int str = (d == 0) ? 1 : ((d == 1) ? N : N * N);
-      const int base = t - id * str;
-#pragma unroll
-      for (int v = 0; v < V; v++) tFb[d][v] = line_T_Dss<N>(lops, id, we + v * nS, base, str);
-      conv_proj_vjp<D>(Us, p, ij[d], tFb[d], a.gamma, Ub);
+        for (int v = 0; v < V; v++) tFb[d][v] = line_T_Dss<N>(lops, id, gb + v * nS, t - id * str, str);
+      }
     }
-    viscous_vjp<D>(
-        Us, p,
-        [&](int j, double *dUj) {
+    __syncthreads();  // the common solution and w are consumed
+    // 3. volume adjoint: F(U, grad) reversed for the cotangent tFb
+    if (valid) {
+      double Us[V];
 #pragma unroll
-          for (int v = 0; v < V; v++) dUj[v] = g_l[(j * V + v) * nS + t];
-        },
-        [&](int v, int j) {
-          double s = 0.0;
+      for (int v = 0; v < V; v++) {
+        Us[v] = u[v * nS + t];
+        Ub[v] = 0.0;
+      }
+      const Prim<D> p = primitives<D>(Us, a.gamma);
 #pragma unroll
-          for (int d1 = 0; d1 < D; d1++) s += tFb[d1][v] * ij[d1][j];
-          return -s;
-        },
-        [&](int j, const double *gbj) {
+      for (int d = 0; d < D; d++) conv_proj_vjp<D>(Us, p, ij[d], tFb[d], a.gamma, Ub);
+      viscous_vjp<D>(
+          Us, p,
+          [&](int j, double *dUj) {
 #pragma unroll
-          for (int v = 0; v < V; v++) gb[(j * V + v) * nS + t] = gbj[v];
-        },
-        a, Ub);
+            for (int v = 0; v < V; v++) dUj[v] = g[v][j];
+          },
+          [&](int v, int j) {
+            double s = 0.0;
+#pragma unroll
+            for (int d1 = 0; d1 < D; d1++) s += tFb[d1][v] * ij[d1][j];
+            return -s;
+          },
+          [&](int j, const double *gbj) {
+#pragma unroll
+            for (int v = 0; v < V; v++) gb[(j * V + v) * nS + t] = gbj[v];
+          },
+          a, Ub);
+    }
   }
-  // 4. the gradient-trace cotangents (k_adj_face, in Gtr) spread back along the normal
-  //    lines, face by face (lines of one face never meet, so the order is fixed)
-#pragma unroll 1
-  for (int q = 0; q < 2 * D; q++) {
-    __syncthreads();
-    if (!valid) continue;
-#pragma unroll
-    for (int k = 0; k < S::FPT; k++) {
-      const int f = t + k * nS;
-      if (f >= nF || f / S::nFF != q) continue;
-      int dim, side, base, str;
-      fpt_info<D, N>(f, dim, side, base, str);
-      const double *lE = tab_lE<N>(lops, side);
+  // 4. the gradient-trace cotangents (k_adj_face, in Gtr) belong to the spts of their normal
+  //    lines: one direction's faces at a time go through LDS and every spt collects the two
+  //    ends of its line (by the face pair's order, so the sums are fixed)
+  {
+    double gv[V][D];
+    if (valid) {
 #pragma unroll
       for (int j = 0; j < D; j++)
 #pragma unroll
-        for (int v = 0; v < V; v++) {
-          const double gt = a.Gtr[((e * D + j) * V + v) * nF + f];
+        for (int v = 0; v < V; v++) gv[v][j] = gb[(j * V + v) * nS + t];
+    }
 #pragma unroll
-          for (int m = 0; m < N; m++) gb[(j * V + v) * nS + base + m * str] += lE[m] * gt;
+    for (int d = 0; d < D; d++) {
+      const int fa = fpt_end<D, N>(0, 0, 0, d, 0) / nFF, fb = fpt_end<D, N>(0, 0, 0, d, 1) / nFF;  // the faces
+      if (d > 0) __syncthreads();  // the previous direction's are consumed
+      if (valid) {
+        for (int i = t; i < 2 * nFF; i += nS) {
+          const int f = (i < nFF) ? fa * nFF + i : fb * nFF + (i - nFF);
+#pragma unroll
+          for (int r = 0; r < D * V; r++) T[r * 2 * nFF + i] = a.Gtr[(e * D * V + r) * nF + f];
+        }
+      }
+      __syncthreads();
+      if (valid) {
+        const int id = (d == 0) ? ia : ((d == 1) ? ib : ic);
+        const double l0 = tab_lE<N>(lops, 0)[id], l1 = tab_lE<N>(lops, 1)[id];
+        const int i0 = fpt_end<D, N>(ia, ib, ic, d, 0) - fa * nFF, i1 = fpt_end<D, N>(ia, ib, ic, d, 1) - fb * nFF + nFF;
+#pragma unroll
+        for (int j = 0; j < D; j++)
+#pragma unroll
+          for (int v = 0; v < V; v++) {
+            const double *Tr = T + (j * V + v) * 2 * nFF;
+            gv[v][j] += l0 * Tr[i0];
+            gv[v][j] += l1 * Tr[i1];
+          }
+      }
+    }
+    // 5. reference-space gradient cotangent: grb[d2][v] = sum_d1 adj[d2][d1] gb[v][d1] / detJ
+    if (valid) {
+      double ij[D][D], detJ;
+      load_metric<D>(a, e, t, nS, ij, detJ, true);
+      const double inv_det = 1.0 / detJ;
+#pragma unroll
+      for (int d2 = 0; d2 < D; d2++)
+#pragma unroll
+        for (int v = 0; v < V; v++) {
+          double s = 0.0;
+#pragma unroll
+          for (int d1 = 0; d1 < D; d1++) s += ij[d2][d1] * gv[v][d1];
+          gb[(d2 * V + v) * nS + t] = s * inv_det;
         }
     }
-  }
-  __syncthreads();
-  // 5. reference-space gradient cotangent: grb[d2][v] = sum_d1 adj[d2][d1] gb[v][d1] / detJ
-  if (valid) {
-    double gv[V][D];
-#pragma unroll
-    for (int j = 0; j < D; j++)
-#pragma unroll
-      for (int v = 0; v < V; v++) gv[v][j] = gb[(j * V + v) * nS + t];
-    const double inv_det = 1.0 / detJ;
-#pragma unroll
-    for (int d2 = 0; d2 < D; d2++)
-#pragma unroll
-      for (int v = 0; v < V; v++) {
-        double s = 0.0;
-#pragma unroll
-        for (int d1 = 0; d1 < D; d1++) s += ij[d2][d1] * gv[v][d1];
-        gb[(d2 * V + v) * nS + t] = s * inv_det;
-      }
   }
   __syncthreads();
   // 6. Dss^T into U; Dsf^T into the common solution's cotangent, split between this
