@@ -1203,17 +1203,15 @@ __global__ __launch_bounds__((Shape<D, N>::kThreads)) void k_divergence_multi(co
 //   k_visc_onesided (gradient, volume flux divergence, owned common fluxes)
 //   -> k_face_correction (oppDiv_fpts Fcomm, both sides).
 
-// Register budget: for hex p=3 four waves per SIMD (<= 128 VGPRs) is what the kernel's
-// LDS allows per CU, and both face phases fit it (Rusanov 110 VGPRs; Roe at the cap) once
-// each gradient line's sum is pinned before the next line is loaded (the value-tied asm
-// fences in the face phase: without them the scheduler issued all the face phase's LDS
-// loads before their FMAs, 168 VGPRs for Roe, 196 for quads at p=4).  Quads at p=4 with
-// Rusanov fit six waves (78-80 VGPRs, no spills; the default allocation took 90 VGPRs,
-// five waves); seven spill.  Other shapes keep the default allocation (at six waves the
-// quad kernels at p = 1..3 spill).
-template <int D, int N, int FC>
+// Register budget: three waves per SIMD for hex p=3.  The kernel's LDS admits 15 waves per CU,
+// but 3.2 per SIMD are in flight on average, with the LDS pipe 70% and the VALU 54% busy
+// (64^3, rocprofv3), so a fourth wave buys nothing: held to 128 VGPRs the Roe kernel spills
+// 10 of them (0.37 GB written and read back per residual; 64^3 residual 1627 us), at 148 it
+// spills none (1488 us).  Rusanov takes 124 either way.  Other shapes keep the default
+// allocation.
+template <int D, int N>
 struct OneSidedWaves {
-  static constexpr int value = (D == 3 && N == 4) ? 4 : ((D == 2 && N == 5 && FC == 0) ? 4 : 1);
+  static constexpr int value = (D == 3 && N == 4) ? 3 : 1;
 };
 
 // SELF: extrapolate the partner traces this element needs from the partner's U (no trace
@@ -1423,7 +1421,7 @@ __device__ __forceinline__ void visc_onesided_block(const double *__restrict__ U
 }
 
 template <int D, int N, int BM, int FC, bool SELF>
-__global__ __launch_bounds__((Shape<D, N>::kThreads)) __attribute__((amdgpu_waves_per_eu(OneSidedWaves<D, N, FC>::value)))
+__global__ __launch_bounds__((Shape<D, N>::kThreads)) __attribute__((amdgpu_waves_per_eu(OneSidedWaves<D, N>::value)))
 void k_visc_onesided(const double *__restrict__ U, double *__restrict__ divF, KArgs a) {
   visc_onesided_block<D, N, BM, FC, SELF>(U, divF, a, xcd_block(blockIdx.x, gridDim.x));
 }
@@ -1432,13 +1430,13 @@ void k_visc_onesided(const double *__restrict__ U, double *__restrict__ divF, KA
 // workgroup, the tile the autotuner picks there): the compiler knows the workgroup is a
 // single wave, so its barriers need no cross-wave synchronisation.
 template <int D, int N, int BM, int FC, bool SELF>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(OneSidedWaves<D, N, FC>::value)))
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(OneSidedWaves<D, N>::value)))
 void k_visc_onesided_w64(const double *__restrict__ U, double *__restrict__ divF, KArgs a) {
   visc_onesided_block<D, N, BM, FC, SELF>(U, divF, a, xcd_block(blockIdx.x, gridDim.x));
 }
 
 template <int D, int N, int BM, int FC>
-__global__ __launch_bounds__((Shape<D, N>::kThreads)) __attribute__((amdgpu_waves_per_eu(OneSidedWaves<D, N, FC>::value)))
+__global__ __launch_bounds__((Shape<D, N>::kThreads)) __attribute__((amdgpu_waves_per_eu(OneSidedWaves<D, N>::value)))
 void k_visc_onesided_multi(const MultiCase *__restrict__ cs, const long *__restrict__ starts, int nc) {
   const int c = find_case(starts, nc, blockIdx.x);
   visc_onesided_block<D, N, BM, FC, true>(cs[c].U, cs[c].out, cs[c].a, (long)blockIdx.x - starts[c]);
