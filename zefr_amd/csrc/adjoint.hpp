@@ -135,6 +135,11 @@ __device__ __forceinline__ void adj_visc_block(const double *__restrict__ U, con
   using L = AdjLds<D, N, true>;
   constexpr int nS = S::nS, nF = S::nF, V = S::V, nFF = S::nFF;
   constexpr int owner = (BM == 2) ? 1 : 0;
+  // hexes with Roe: what must outlive the face adjoint waits in global memory (the partner's
+  // trace in Utr at this element's own point, the volume adjoint's part in vout) instead of
+  // in registers, which the Roe reverse sweep fills: left to the compiler they are spilled,
+  // which costs more (VJP of 32^3 hexes p=3 431 us spilled, 419 this way)
+  constexpr bool kPark = D == 3 && FC == 1;
   extern __shared__ double lds[];
   const int EB = a.EB;
   double *lops = lds;
@@ -156,9 +161,9 @@ __device__ __forceinline__ void adj_visc_block(const double *__restrict__ U, con
   double wr[V];
 #pragma unroll
   for (int v = 0; v < V; v++) wr[v] = valid ? w[(e * V + v) * nS + t] : 0.0;
-  const unsigned mask = valid ? owned_faces<D, N>(a.nbr + e * nF, owner) : 0u;
-  const unsigned owned = face_list<D>(mask), unowned = face_list<D>(~mask);
-  const int cnt = __popc(mask) * nFF;
+  unsigned mask = valid ? owned_faces<D, N>(a.nbr + e * nF, owner) : 0u;
+  unsigned owned = face_list<D>(mask), unowned = face_list<D>(~mask);
+  int cnt = __popc(mask) * nFF;
   // the element's last pass starts at work item 'last' (0 unless more than nS points are owned)
   const int last = (cnt > nS) ? ((cnt - 1) / nS) * nS : 0;
   const int klast = t + last;
@@ -168,7 +173,10 @@ __device__ __forceinline__ void adj_visc_block(const double *__restrict__ U, con
     const int f = list_fpt<D, N>(owned, klast);
     owned_partner_trace<D, N>(U, a, e, f, cp);
 #pragma unroll
-    for (int v = 0; v < V; v++) c[v * nF + f] = cp[v];
+    for (int v = 0; v < V; v++) {
+      c[v * nF + f] = cp[v];
+      if (kPark) a.Utr[(e * V + v) * nF + f] = cp[v];
+    }
   }
 #pragma unroll 1
   for (int k = t; k < last; k += nS) {
@@ -203,7 +211,7 @@ __device__ __forceinline__ void adj_visc_block(const double *__restrict__ U, con
   __syncthreads();
   // 2. forward physical gradient at every spt, into the region of c; tFb[d1] = Dss^T w along
   //    the d1 lines
-  double Ub[V], tFb[D][V];
+  double Ub[kPark ? 1 : V], tFb[D][V];
   {
     double ij[D][D], detJ, g[V][D];
     if (valid) {
@@ -227,15 +235,15 @@ __device__ __forceinline__ void adj_visc_block(const double *__restrict__ U, con
     __syncthreads();  // w is consumed
     // 3. volume adjoint: F(U, grad) reversed for the cotangent tFb
     if (valid) {
-      double Us[V];
+      double Us[V], Usb[V];
 #pragma unroll
       for (int v = 0; v < V; v++) {
         Us[v] = u[v * nS + t];
-        Ub[v] = 0.0;
+        Usb[v] = 0.0;
       }
       const Prim<D> p = primitives<D>(Us, a.gamma);
 #pragma unroll
-      for (int d = 0; d < D; d++) conv_proj_vjp<D>(Us, p, ij[d], tFb[d], a.gamma, Ub);
+      for (int d = 0; d < D; d++) conv_proj_vjp<D>(Us, p, ij[d], tFb[d], a.gamma, Usb);
       // tF[d1] -= T . adj[d1]: cotangent on T[v][j] is -sum_d1 tFb[d1][v] adj[d1][j]
       viscous_vjp<D>(
           Us, p,
@@ -253,7 +261,12 @@ __device__ __forceinline__ void adj_visc_block(const double *__restrict__ U, con
 #pragma unroll
             for (int v = 0; v < V; v++) gb[(j * V + v) * nS + t] = gbj[v];
           },
-          a, Ub);
+          a, Usb);
+#pragma unroll
+      for (int v = 0; v < V; v++) {
+        if (kPark) vout[(e * V + v) * nS + t] = Usb[v];
+        else Ub[kPark ? 0 : v] = Usb[v];
+      }
     }
   }
   // 4. face adjoint at the owned points.  An owned point's gradient cotangent belongs to the
@@ -281,7 +294,7 @@ __device__ __forceinline__ void adj_visc_block(const double *__restrict__ U, con
 #pragma unroll
         for (int v = 0; v < V; v++) {
           Uo[v] = line_extrap<N>(lE, u + v * nS, base, str);
-          Up[v] = fin ? cp[v] : a.Utr[(e * V + v) * nF + f];
+          Up[v] = (fin && !kPark) ? cp[v] : a.Utr[(e * V + v) * nF + f];
         }
         owned_flux_vjp<D, N, true, BM, FC>(a, Wtr, e, f, n, Uo, Up, Uob, Upb, Gb);
 #pragma unroll
@@ -335,6 +348,12 @@ __device__ __forceinline__ void adj_visc_block(const double *__restrict__ U, con
     }
   }
   __syncthreads();
+  if (kPark) {  // formed again rather than held (or spilled) across the face adjoint
+    asm volatile("" : "+v"(mask));
+    owned = face_list<D>(mask);
+    unowned = face_list<D>(~mask);
+    cnt = __popc(mask) * nFF;
+  }
   // 5. each spt collects the gradient-trace cotangents of the owned ends of its lines, then
   //    reference-space gradient cotangent: grb[d2][v] = sum_d1 adj[d2][d1] gb[v][d1] / detJ
   //    (the metric read again here: held across the face adjoint it takes registers the
@@ -380,13 +399,16 @@ __device__ __forceinline__ void adj_visc_block(const double *__restrict__ U, con
   __syncthreads();
   // 6. Dss^T into U, Dsf^T into the common solution's cotangent: the partner's trace at
   //    owned points (Xtr), this element's trace elsewhere
+  double vb[V];
   if (valid) {
+#pragma unroll
+    for (int v = 0; v < V; v++) vb[v] = kPark ? vout[(e * V + v) * nS + t] : Ub[kPark ? 0 : v];
 #pragma unroll
     for (int d = 0; d < D; d++) {
       const int id = (d == 0) ? ia : ((d == 1) ? ib : ic);
       const int str = (d == 0) ? 1 : ((d == 1) ? N : N * N);
 #pragma unroll
-      for (int v = 0; v < V; v++) Ub[v] += line_T_Dss<N>(lops, id, gb + (d * V + v) * nS, t - id * str, str);
+      for (int v = 0; v < V; v++) vb[v] += line_T_Dss<N>(lops, id, gb + (d * V + v) * nS, t - id * str, str);
     }
     auto dsf = [&](int f, double *cb) {
       int dim, side, base, str;
@@ -431,10 +453,10 @@ __device__ __forceinline__ void adj_visc_block(const double *__restrict__ U, con
     const double l0 = tab_lE<N>(lops, 0)[id], l1 = tab_lE<N>(lops, 1)[id];
     const int f0 = fpt_end<D, N>(ia, ib, ic, d, 0), f1 = fpt_end<D, N>(ia, ib, ic, d, 1);
 #pragma unroll
-    for (int v = 0; v < V; v++) Ub[v] += l0 * to[v * nF + f0] + l1 * to[v * nF + f1];
+    for (int v = 0; v < V; v++) vb[v] += l0 * to[v * nF + f0] + l1 * to[v * nF + f1];
   }
 #pragma unroll
-  for (int v = 0; v < V; v++) vout[(e * V + v) * nS + t] = Ub[v];
+  for (int v = 0; v < V; v++) vout[(e * V + v) * nS + t] = vb[v];
 }
 
 // Euler: the volume adjoint, the face adjoint at the owned points (slot 0), and E^T.
