@@ -466,6 +466,20 @@ int zfr_pmg_transfer(int nDims, int nVars, long nEles, int n_in, int n_out, cons
  * src/aux_kernels.cu:143-205); z may alias x or y. */
 int zfr_axpby(long n, double a, const double *x, double b, const double *y, double *z, void *stream);
 
+/* Stage arithmetic of a classical RK44 step of dU/dt = -R(U)/detJ on fields [nEles][nVars][nSpts]
+ * with a caller-supplied detJ [nEles][nSpts] (src/solver.cpp:713-735), and its reverse; each
+ * operation is rounded on its own.  With k = -R/detJ:
+ *   stage:     X = U + c k(R)
+ *   final:     Y = U + dt (k(R[0])/6 + k(R[1])/3 + k(R[2])/3 + k(R[3])/6); R is a host array
+ *   cotangent: w = (cg g - cq q)/detJ (q NULL: 0; skipped when w is NULL) and
+ *              acc_out = acc_in - q (skipped when acc_out is NULL; acc_out may be acc_in) */
+int zfr_rk4_stage(long nEles, int nVars, int nSpts, const double *U, const double *R, const double *detJ, double c,
+                  double *X, void *stream);
+int zfr_rk4_final(long nEles, int nVars, int nSpts, const double *U, const double *const *R, const double *detJ,
+                  double dt, double *Y, void *stream);
+int zfr_rk4_cotangent(long nEles, int nVars, int nSpts, const double *g, const double *q, const double *detJ,
+                      double cg, double cq, double *w, const double *acc_in, double *acc_out, void *stream);
+
 /* ---------------------------------------------------------------- host physics --- */
 
 /* Physical parameters of the pointwise fluxes (InputStruct fields of the same names). */

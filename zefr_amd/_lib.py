@@ -166,6 +166,9 @@ SIGNATURES = {
     "zfr_rk_final_source": (_I, [C.POINTER(EleDesc), _P, _P, _P, _P, _DP, _I, C.c_double, _P]),
     "zfr_pmg_transfer": (_I, [_I, _I, C.c_long, _I, _I, _P, C.c_double, _P, C.c_double, _P, _P]),
     "zfr_axpby": (_I, [C.c_long, C.c_double, _P, C.c_double, _P, _P, _P]),
+    "zfr_rk4_stage": (_I, [C.c_long, _I, _I, _P, _P, _P, C.c_double, _P, _P]),
+    "zfr_rk4_final": (_I, [C.c_long, _I, _I, _P, C.POINTER(_P), _P, C.c_double, _P, _P]),
+    "zfr_rk4_cotangent": (_I, [C.c_long, _I, _I, _P, _P, _P, C.c_double, C.c_double, _P, _P, _P, _P]),
     "zfr_host_point_flux": (_I, [_I, C.POINTER(ZfrPhys), _DP, _DP, _DP]),
     "zfr_host_point_flux_vjp": (_I, [_I, C.POINTER(ZfrPhys), _DP, _DP, _DP, _DP, _DP]),
     "zfr_host_common_flux": (_I, [_I, C.POINTER(ZfrPhys), _I, _DP, _DP, _DP, _DP, _DP, C.c_double, _DP]),

@@ -17,6 +17,8 @@ the backward pass (torch.utils.checkpoint), so memory holds one state per block.
 
 from __future__ import annotations
 
+import ctypes as C
+
 import numpy as np
 import torch
 
@@ -104,10 +106,80 @@ def device_field(z, name):
     return torch.from_numpy(np.ascontiguousarray(t)).to("cuda")
 
 
+class RK4Step(torch.autograd.Function):
+    """One RK44 step with its stage combinations as one kernel each (zfr_rk4_stage, _final) and
+    its reverse sweep as four residual VJPs with one kernel between them (zfr_rk4_cotangent).
+    The values are those of the tensor expressions in rk4_step.  Saves the four stage states,
+    as those expressions do."""
+
+    @staticmethod
+    def forward(ctx, U, z, dt, detJ):
+        from ._lib import check, lib
+        X = [U.detach().contiguous()]
+        E, V, nS = X[0].shape
+        dj = detJ.data_ptr()
+        R = []
+        for c in (0.5 * dt, 0.5 * dt, dt, None):
+            R.append(z.residual_at(X[-1]))
+            if c is None:
+                break
+            X.append(torch.empty_like(X[0]))
+            check(lib().zfr_rk4_stage(E, V, nS, X[0].data_ptr(), R[-1].data_ptr(), dj, c, X[-1].data_ptr(), _stream()))
+        Y = torch.empty_like(X[0])
+        ptrs = (C.c_void_p * 4)(*[r.data_ptr() for r in R])
+        check(lib().zfr_rk4_final(E, V, nS, X[0].data_ptr(), ptrs, dj, dt, Y.data_ptr(), _stream()))
+        ctx.z, ctx.dt = z, dt
+        ctx.save_for_backward(U, X[1], X[2], X[3], detJ)
+        return Y
+
+    @staticmethod
+    def backward(ctx, g):
+        U, X2, X3, X4, detJ = ctx.saved_tensors
+        with torch.no_grad():
+            v = RK4Step._reverse(ctx.z, ctx.dt, detJ, (U.contiguous(), X2, X3, X4), g.contiguous())
+        if torch.is_grad_enabled():  # create_graph: v depends on g through the identity; the VJPs are constants
+            v = g + (v - g.detach())
+        return v, None, None, None
+
+    @staticmethod
+    def _reverse(z, dt, detJ, X, g):
+        """dL/dU for g = dL/dY.  With q_s = (dR/dX_s)^T w_s and w_s the cotangent of stage s's
+        slope over detJ: w_4 = dt/6 g, w_3 = dt/3 g - dt q_4, w_2 = dt/3 g - dt/2 q_3,
+        w_1 = dt/6 g - dt/2 q_2 (each over detJ) and dL/dU = g - q_4 - q_3 - q_2 - q_1."""
+        from ._lib import check, lib
+        E, V, nS = g.shape
+        w, acc, q = torch.empty_like(g), torch.empty_like(g), None
+        for s, cg, cq in ((3, dt / 6, 0.0), (2, dt / 3, dt), (1, dt / 3, 0.5 * dt), (0, dt / 6, 0.5 * dt)):
+            check(lib().zfr_rk4_cotangent(E, V, nS, g.data_ptr(), q.data_ptr() if q is not None else None,
+                                          detJ.data_ptr(), cg, cq, w.data_ptr(),
+                                          (g if s == 2 else acc).data_ptr() if q is not None else None,
+                                          acc.data_ptr() if q is not None else None, _stream()))
+            q = z.residual_vjp(X[s], w, q)
+        check(lib().zfr_rk4_cotangent(E, V, nS, None, q.data_ptr(), None, 0.0, 0.0, None, acc.data_ptr(),
+                                      acc.data_ptr(), _stream()))
+        return acc
+
+
+def _stream():
+    return torch.cuda.current_stream().cuda_stream
+
+
+def _fusable(z, U, dt, detJ, mu):
+    """Whether RK4Step covers the call: a number for dt, constant viscosity, and a plain
+    contiguous detJ field that is not differentiated.  Everything else takes the tensor
+    expressions (U itself is checked by the residual either way)."""
+    return (mu is None and type(dt) in (int, float) and type(U) in (torch.Tensor, torch.nn.Parameter)
+            and type(detJ) is torch.Tensor and U.dim() == 3 and detJ.shape == (U.shape[0], 1, U.shape[2])
+            and detJ.dtype == torch.float64 and U.dtype == torch.float64 and detJ.is_cuda and U.is_cuda
+            and detJ.device == U.device and detJ.is_contiguous() and not detJ.requires_grad)
+
+
 def rk4_step(z, U, dt, detJ=None, mu=None):
     """One classical RK4 step of dU/dt = -R(U)/detJ (src/solver.cpp:2865-3097)."""
     if detJ is None:
         detJ = device_field(z, "jaco_det_spts")
+    if _fusable(z, U, dt, detJ, mu):
+        return RK4Step.apply(U, z, dt, detJ)
     f = lambda X: -residual(z, X, mu) / detJ  # noqa: E731
     k1 = f(U)
     k2 = f(U + 0.5 * dt * k1)

@@ -119,6 +119,68 @@ __global__ __launch_bounds__(kMaxThreads) void k_axpby(double *z, double a, cons
     z[i] = a * x[i] + b * y[i];
 }
 
+// The stage arithmetic of a differentiated RK44 step (autograd.rk4_step) on [E][V][nS]
+// fields with the caller's detJ [E][nS], one thread per point: bound by memory, a pass per
+// stage instead of one per tensor expression (16^3 hexes p=3, step and gradient: about 60
+// elementwise launches less).  Products and sums are rounded one by one, as the tensor
+// expressions they stand for.
+//   stage    X = U + c k(R),                    k(R) = -R / detJ
+//   final    Y = U + dt (k1/6 + k2/3 + k3/3 + k4/6)
+//   reverse  w = (cg g - cq q) / detJ and acc_out = acc_in - q
+template <int V>
+__global__ __launch_bounds__(kMaxThreads) void k_rk4_stage(const double *__restrict__ U, const double *__restrict__ R,
+                                                           const double *__restrict__ detJ, double c,
+                                                           double *__restrict__ X, long pts, int nS) {
+#pragma clang fp contract(off)
+  for (long p = (long)blockIdx.x * blockDim.x + threadIdx.x; p < pts; p += (long)gridDim.x * blockDim.x) {
+    const long i0 = p + (p / nS) * (V - 1) * nS;
+    const double dj = detJ[p];
+#pragma unroll
+    for (int v = 0; v < V; v++) X[i0 + v * nS] = U[i0 + v * nS] + c * (-R[i0 + v * nS] / dj);
+  }
+}
+
+struct Rk4R {
+  const double *R[4];
+};
+
+template <int V>
+__global__ __launch_bounds__(kMaxThreads) void k_rk4_final(const double *__restrict__ U, Rk4R r,
+                                                           const double *__restrict__ detJ, double dt,
+                                                           double *__restrict__ Y, long pts, int nS) {
+#pragma clang fp contract(off)
+  for (long p = (long)blockIdx.x * blockDim.x + threadIdx.x; p < pts; p += (long)gridDim.x * blockDim.x) {
+    const long i0 = p + (p / nS) * (V - 1) * nS;
+    const double dj = detJ[p];
+#pragma unroll
+    for (int v = 0; v < V; v++) {
+      const long i = i0 + v * nS;
+      const double k1 = -r.R[0][i] / dj, k2 = -r.R[1][i] / dj, k3 = -r.R[2][i] / dj, k4 = -r.R[3][i] / dj;
+      Y[i] = U[i] + dt * (((k1 * (1.0 / 6.0) + k2 * (1.0 / 3.0)) + k3 * (1.0 / 3.0)) + k4 * (1.0 / 6.0));
+    }
+  }
+}
+
+template <int V>
+__global__ __launch_bounds__(kMaxThreads) void k_rk4_cotangent(const double *__restrict__ g,
+                                                               const double *__restrict__ q,
+                                                               const double *__restrict__ detJ, double cg, double cq,
+                                                               double *__restrict__ w, const double *acc_in,
+                                                               double *acc_out, long pts, int nS) {
+#pragma clang fp contract(off)
+  for (long p = (long)blockIdx.x * blockDim.x + threadIdx.x; p < pts; p += (long)gridDim.x * blockDim.x) {
+    const long i0 = p + (p / nS) * (V - 1) * nS;
+    const double dj = w ? detJ[p] : 1.0;
+#pragma unroll
+    for (int v = 0; v < V; v++) {
+      const long i = i0 + v * nS;
+      const double qi = q ? q[i] : 0.0;
+      if (w) w[i] = (cg * g[i] - cq * qi) / dj;
+      if (acc_out) acc_out[i] = acc_in[i] - qi;
+    }
+  }
+}
+
 __device__ __forceinline__ double wave_reduce(double x, int type) {
   for (int off = warpSize / 2; off > 0; off >>= 1) {
     const double y = __shfl_down(x, off);
@@ -542,6 +604,52 @@ int zfr_axpby(long n, double a, const double *x, double b, const double *y, doub
                      y, n);
   return zfr::check_hip(hipGetLastError(), "zfr_axpby");
 }
+
+namespace {
+int rk4_checks(long nEles, int nVars, int nSpts, const char *who) {
+  if (int rc = zk::refuse_while_recording(who)) return rc;
+  if (nVars != 4 && nVars != 5) return zfr::fail(std::string(who) + ": nVars must be 4 or 5");
+  if (nEles < 0 || nSpts < 1) return zfr::fail(std::string(who) + ": bad sizes");
+  return 0;
+}
+}  // namespace
+
+#define ZK_RK4(K_, ...)                                                                                            \
+  do {                                                                                                             \
+    const long pts = nEles * nSpts;                                                                                \
+    const dim3 grid(zk::grid_for(pts)), block(zk::kMaxThreads);                                                    \
+    if (nVars == 4) hipLaunchKernelGGL((zk::K_<4>), grid, block, 0, (hipStream_t)stream, __VA_ARGS__, pts, nSpts); \
+    else hipLaunchKernelGGL((zk::K_<5>), grid, block, 0, (hipStream_t)stream, __VA_ARGS__, pts, nSpts);            \
+  } while (0)
+
+int zfr_rk4_stage(long nEles, int nVars, int nSpts, const double *U, const double *R, const double *detJ, double c,
+                  double *X, void *stream) {
+  if (int rc = rk4_checks(nEles, nVars, nSpts, "zfr_rk4_stage")) return rc;
+  if (nEles == 0) return 0;
+  if (!U || !R || !detJ || !X) return zfr::fail("zfr_rk4_stage: missing buffer");
+  ZK_RK4(k_rk4_stage, U, R, detJ, c, X);
+  return zfr::check_hip(hipGetLastError(), "zfr_rk4_stage");
+}
+
+int zfr_rk4_final(long nEles, int nVars, int nSpts, const double *U, const double *const *R, const double *detJ,
+                  double dt, double *Y, void *stream) {
+  if (int rc = rk4_checks(nEles, nVars, nSpts, "zfr_rk4_final")) return rc;
+  if (nEles == 0) return 0;
+  if (!U || !R || !R[0] || !R[1] || !R[2] || !R[3] || !detJ || !Y) return zfr::fail("zfr_rk4_final: missing buffer");
+  const zk::Rk4R r = {{R[0], R[1], R[2], R[3]}};
+  ZK_RK4(k_rk4_final, U, r, detJ, dt, Y);
+  return zfr::check_hip(hipGetLastError(), "zfr_rk4_final");
+}
+
+int zfr_rk4_cotangent(long nEles, int nVars, int nSpts, const double *g, const double *q, const double *detJ,
+                      double cg, double cq, double *w, const double *acc_in, double *acc_out, void *stream) {
+  if (int rc = rk4_checks(nEles, nVars, nSpts, "zfr_rk4_cotangent")) return rc;
+  if (nEles == 0) return 0;
+  if ((w && (!g || !detJ)) || (acc_out && (!acc_in || !q))) return zfr::fail("zfr_rk4_cotangent: missing buffer");
+  ZK_RK4(k_rk4_cotangent, g, q, detJ, cg, cq, w, acc_in, acc_out);
+  return zfr::check_hip(hipGetLastError(), "zfr_rk4_cotangent");
+}
+#undef ZK_RK4
 
 }  // extern "C"
 
