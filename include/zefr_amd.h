@@ -201,6 +201,11 @@ int zefr_residual_at(zefr_t *z, const double *U, double *divF, void *stream);
  * null stream): the residual's vector-Jacobian product (new; no reference counterpart).
  * Euler, or Navier-Stokes with LDG beta = +-1/2.  Same scratch rule as residual_at. */
 int zefr_residual_vjp(zefr_t *z, const double *U, const double *w, double *v, void *stream);
+/* The same on arrays of a stated shape, which must be the solver's [nEles][nVars][nSpts]; they
+ * wait for the solver's own stream (on the host) before they launch on `stream`. */
+int zefr_residual_tensor(zefr_t *z, const double *U, double *divF, long nEles, long nVars, long nSpts, void *stream);
+int zefr_residual_vjp_tensor(zefr_t *z, const double *U, const double *w, double *v, long nEles, long nVars,
+                             long nSpts, void *stream);
 /* p-multigrid (PMGrid, include/multigrid.hpp:17-44): with p_multi set, setup_solver builds
  * the coarse FRSolvers of mg_levels (PMGrid::setup, src/multigrid.cpp:18-103) and do_step
  * runs PMGrid::cycle (src/multigrid.cpp:263-333) instead of one update.  The per-level

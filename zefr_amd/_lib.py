@@ -119,6 +119,8 @@ SIGNATURES = {
     "zefr_time_residual_kernels": (_I, [_P, _I, _DP]),
     "zefr_residual_at": (_I, [_P, _P, _P, _P]),
     "zefr_residual_vjp": (_I, [_P, _P, _P, _P, _P]),
+    "zefr_residual_tensor": (_I, [_P, _P, _P, C.c_long, C.c_long, C.c_long, _P]),
+    "zefr_residual_vjp_tensor": (_I, [_P, _P, _P, _P, C.c_long, C.c_long, C.c_long, _P]),
     "zefr_pmg_copy_state": (_I, [_P, _I, _I, _DP, C.c_long, _I]),
     "zefr_batch_create": (_P, [C.POINTER(_P), _I]),
     "zefr_batch_residual": (_I, [_P]),

@@ -386,6 +386,31 @@ int zefr_residual_vjp(zefr_t *z, const double *U, const double *w, double *v, vo
   return zfr::guard([&] { z->s().residual_vjp(U, w, v, (hipStream_t)stream); });
 }
 
+// The tensor forms: the caller's shape checked against the solver's, the solver's own
+// (non-blocking) stream waited for, then the launches, in one call.
+static void ready_for_tensors(zfr::FRSolver &s, long nEles, long nVars, long nSpts, const char *who) {
+  if (!s.device_ready) zfr::raise("solver is not set up on the device (call setup_solver)");
+  const zfr::Elements &e = *s.eles;
+  if (nEles != e.nEles || nVars != e.nVars || nSpts != e.nSpts)
+    zfr::raise(std::string(who) + ": the tensors' shape is not the solver's [nEles][nVars][nSpts]");
+  s.synchronize();
+}
+
+int zefr_residual_tensor(zefr_t *z, const double *U, double *divF, long nEles, long nVars, long nSpts, void *stream) {
+  return zfr::guard([&] {
+    ready_for_tensors(z->s(), nEles, nVars, nSpts, "zefr_residual_tensor");
+    z->s().residual_at(U, divF, (hipStream_t)stream);
+  });
+}
+
+int zefr_residual_vjp_tensor(zefr_t *z, const double *U, const double *w, double *v, long nEles, long nVars,
+                             long nSpts, void *stream) {
+  return zfr::guard([&] {
+    ready_for_tensors(z->s(), nEles, nVars, nSpts, "zefr_residual_vjp_tensor");
+    z->s().residual_vjp(U, w, v, (hipStream_t)stream);
+  });
+}
+
 int zefr_set_tile(zefr_t *z, int eles_per_block) {
   return zfr::guard([&] {
     if (eles_per_block < 0) zfr::raise("tile must be >= 0");

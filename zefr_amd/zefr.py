@@ -34,6 +34,16 @@ _STR_FIELDS = {"dt_scheme", "meshfile", "output_prefix", "spt_type", "mg_cycle",
 _LEVEL_FIELDS = ("mg_levels", "mg_steps")
 
 
+def _torch():
+    import torch
+    return torch
+
+
+def current_stream():
+    """torch's current stream as a raw handle."""
+    return _torch().cuda.current_stream().cuda_stream
+
+
 class InputStruct:
     """Attribute view of the library's ``zefr_input_t`` (InputStruct field names)."""
 
@@ -248,30 +258,55 @@ class Zefr:
             raise ValueError(f"expected a contiguous float64 device tensor of shape {shape} "
                              "(the device layout [nEles][nVars][nSpts])")
 
+    def _ready(self, *ts):
+        """Whether the tensors are plain contiguous float64 device tensors of one 3D shape; the
+        library itself compares that shape with the solver's."""
+        torch = _torch()
+        s = ts[0].shape if type(ts[0]) is torch.Tensor else None
+        for t in ts:
+            if not (type(t) is torch.Tensor and t.dtype is torch.float64 and t.is_cuda and t.shape == s
+                    and t.is_contiguous()):
+                return False
+        return len(s) == 3
+
     # Both run on torch's current stream (torch and the library share one HIP runtime, see
-    # _lib._init_torch_first), ordered with the surrounding torch work.
+    # _lib._init_torch_first), ordered with the surrounding torch work, after waiting for the
+    # solver's own stream, which is non-blocking and shares the scratch.
     def residual_at(self, U, out=None):
         """R(U) = divF for the device state U (torch float64 [nEles][nVars][nSpts]),
         without touching the solver's own state."""
-        import torch
+        if out is None:
+            self._tensor_ok(U)
+            out = _torch().empty_like(U)
+        if self._ready(U, out):
+            s = U.shape
+            rc = lib().zefr_residual_tensor(self._h, U.data_ptr(), out.data_ptr(), s[0], s[1], s[2],
+                                            current_stream())
+            if rc == 0:
+                return out
         self._tensor_ok(U)
-        out = torch.empty_like(U) if out is None else out
         self._tensor_ok(out)
-        self.synchronize()  # the solver's own stream is non-blocking; it shares the scratch
-        st = torch.cuda.current_stream().cuda_stream
-        check(lib().zefr_residual_at(self._h, U.data_ptr(), out.data_ptr(), st))
+        self.synchronize()
+        check(lib().zefr_residual_at(self._h, U.data_ptr(), out.data_ptr(), current_stream()))
         return out
 
     def residual_vjp(self, U, w, out=None):
         """v = (dR/dU)^T w at U (device tensors in the device layout)."""
-        import torch
+        if out is None:
+            self._tensor_ok(U)
+            self._tensor_ok(w)
+            out = _torch().empty_like(U)
+        if self._ready(U, w, out):
+            s = U.shape
+            rc = lib().zefr_residual_vjp_tensor(self._h, U.data_ptr(), w.data_ptr(), out.data_ptr(), s[0], s[1],
+                                                s[2], current_stream())
+            if rc == 0:
+                return out
         self._tensor_ok(U)
         self._tensor_ok(w)
-        out = torch.empty_like(U) if out is None else out
         self._tensor_ok(out)
-        self.synchronize()  # the solver's own stream is non-blocking; it shares the scratch
-        st = torch.cuda.current_stream().cuda_stream
-        check(lib().zefr_residual_vjp(self._h, U.data_ptr(), w.data_ptr(), out.data_ptr(), st))
+        self.synchronize()
+        check(lib().zefr_residual_vjp(self._h, U.data_ptr(), w.data_ptr(), out.data_ptr(), current_stream()))
         return out
 
     # -- data access (src/zefr.cpp:560-650)
