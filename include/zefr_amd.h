@@ -276,7 +276,8 @@ typedef struct zfr_ele_desc {
   double *Utr;                     /* [E][V][nF] solution trace (scratch)                */
   double *Gtr;                     /* [E][D][V][nF] gradient trace (scratch, viscous)    */
   double *Ftr;                     /* [E][V][nF] common normal flux at the flux points
-                                      whose side owns it (scratch, LDG beta = +-1/2)     */
+                                      whose side owns it (scratch, LDG beta = +-1/2), or each
+                                      side's share of it (zfr_both_sides_flux)           */
   int fconv_type;                  /* convective common flux: 0 Rusanov, 2 Roe           */
 } zfr_ele_desc_t;
 
@@ -401,6 +402,15 @@ typedef struct zfr_rk_args {
   double *prolong_out;
 } zfr_rk_args_t;
 int zfr_face_correction_rk(const zfr_ele_desc_t *d, double *divF, const zfr_rk_args_t *rk, void *stream);
+/* The two launches of a viscous residual with LDG beta other than +-1/2 (both sides' gradients
+ * in each common flux, src/faces.cpp:1476-1614), as zfr_gradient_flux and zfr_face_correction
+ * are for beta = +-1/2: the first writes the volume part of divF and this side's share of the
+ * common flux at every flux point to d->Ftr, the second adds both sides' shares.  The partner
+ * traces come from the partners' U, or (traced != 0) from d->Utr at every flux point, as
+ * zfr_extrapolate or a fused update's trace_out writes it.  rk: an epilogue as in
+ * zfr_face_correction_rk (trace_out takes every flux point and may be d->Utr), or NULL. */
+int zfr_both_sides_flux(const zfr_ele_desc_t *d, const double *U, double *divF, int traced, void *stream);
+int zfr_both_sides_correction(const zfr_ele_desc_t *d, double *divF, const zfr_rk_args_t *rk, void *stream);
 int zfr_divergence_rk(const zfr_ele_desc_t *d, const double *U, double *divF, const zfr_rk_args_t *rk,
                       void *stream);
 /* Vector-Jacobian product of one residual (new; no reference counterpart): for the state

@@ -168,6 +168,8 @@ class FRSolver {
   void synchronize();
   int autotune(int reps);
   bool onesided() const;  // viscous with LDG beta = +-1/2: one-sided gradient path
+  void viscous_flux(const zfr_ele_desc_t &d, const double *U, double *divF, bool traced, hipStream_t st);
+  void last_launch(const zfr_ele_desc_t &d, const double *U, double *divF, const zfr_rk_args_t *rk, hipStream_t st);
   void time_kernels(int reps, double *ms_out);
   // The residual of an arbitrary device state U [E][V][nS] into divF (same layout) on the
   // caller's stream st (nullptr: the null stream), with the kernels of compute_residual;

@@ -436,7 +436,7 @@ int rk_fused(zk::Op op, const zfr_ele_desc_t *d, const double *U, double *divF, 
       return zfr::fail("RK fusion: restriction needs restrict_A, restrict_U and restrict_divF");
     if (r->restrict_n < 1 || r->restrict_n > d->order + 1)
       return zfr::fail("RK fusion: restrict_n must be in 1..order+1");
-    if (op == zk::Op::FaceCorr && !r->restrict_src)
+    if ((op == zk::Op::FaceCorr || op == zk::Op::FaceCorrBoth) && !r->restrict_src)
       return zfr::fail("RK fusion: the face correction restricts U from restrict_src");
   }
   if (prol) {
@@ -496,7 +496,7 @@ int rk_fused(zk::Op op, const zfr_ele_desc_t *d, const double *U, double *divF, 
   int rc = need_geometry(d);
   if (!rc && reads_tr) rc = need(d->Utr, "Utr");
   if (!rc && op == zk::Op::Div && d->viscous && d->ldg_b != 0.5 && d->ldg_b != -0.5) rc = need(d->Gtr, "Gtr");
-  if (!rc && op == zk::Op::FaceCorr) rc = need(d->Ftr, "Ftr");
+  if (!rc && (op == zk::Op::FaceCorr || op == zk::Op::FaceCorrBoth)) rc = need(d->Ftr, "Ftr");
   if (rc) return rc;
   if (update && (r->nStages < 1 || r->nStages > zk::kMaxRkStages || r->stage < 0 || r->stage >= r->nStages))
     return zfr::fail("RK fusion: stage out of range");
@@ -509,6 +509,24 @@ int rk_fused(zk::Op op, const zfr_ele_desc_t *d, const double *U, double *divF, 
 }  // namespace
 
 extern "C" {
+
+int zfr_both_sides_flux(const zfr_ele_desc_t *d, const double *U, double *divF, int traced, void *stream) {
+  int rc = need_geometry(d);
+  if (!rc) rc = need_arg(U, "U");
+  if (!rc) rc = need_arg(divF, "divF");
+  if (!rc && traced) rc = need(d->Utr, "Utr");
+  if (!rc) rc = need(d->Ftr, "Ftr");
+  if (rc) return rc;
+  return zk::dispatch(traced ? zk::Op::BothSidesFromTrace : zk::Op::BothSides, d, U, divF, (hipStream_t)stream);
+}
+
+int zfr_both_sides_correction(const zfr_ele_desc_t *d, double *divF, const zfr_rk_args_t *rk, void *stream) {
+  if (int rc = need_geometry(d)) return rc;
+  if (int rc = need_arg(divF, "divF")) return rc;
+  if (rk) return rk_fused(zk::Op::FaceCorrBoth, d, nullptr, divF, rk, (hipStream_t)stream);
+  if (int rc = need(d->Ftr, "Ftr")) return rc;
+  return zk::dispatch(zk::Op::FaceCorrBoth, d, nullptr, divF, (hipStream_t)stream);
+}
 
 int zfr_face_correction_rk(const zfr_ele_desc_t *d, double *divF, const zfr_rk_args_t *rk, void *stream) {
   if (int rc = need_geometry(d)) return rc;
@@ -825,10 +843,16 @@ int zfr_multi_create(const zfr_ele_desc_t *descs, const double *const *U, double
       phase[1][{Op::OneSided, mixed ? 0 : D, mixed ? 0 : N, 1, bm, fc}].push_back(i);  // extrapolates the partner traces itself
       phase[2][{Op::FaceCorr, mixed ? 0 : D, mixed ? 0 : N, 1, bm, 0}].push_back(i);
     } else {
+      // general beta: the trace, then the both-sides pair (its shares of the common flux go
+      // to the Gtr buffer, the scratch such a case has always brought)
       if (visc && !d->Gtr) return zfr::fail("zfr_multi_create: the general LDG path needs Gtr");
-      if (visc) phase[0][{Op::Extrap, D, N, 0, 0, 0}].push_back(i);  // Euler: extrapolated in the divergence
-      if (visc) phase[1][{Op::Grad, D, N, 1, 0, 0}].push_back(i);
-      const bool own = visc || N > zk::kMixedMaxN;
+      if (visc) {
+        phase[0][{Op::Extrap, D, N, 0, 0, 0}].push_back(i);
+        phase[1][{Op::BothSidesFromTrace, D, N, 1, 0, fc}].push_back(i);
+        phase[2][{Op::FaceCorrBoth, D, N, 1, 0, 0}].push_back(i);
+        continue;
+      }
+      const bool own = N > zk::kMixedMaxN;  // Euler: the partner traces are extrapolated in the divergence
       phase[2][{Op::Div, own ? D : 0, own ? N : 0, visc, bm, fc}].push_back(i);
     }
   }
@@ -882,9 +906,9 @@ int zfr_multi_create(const zfr_ele_desc_t *descs, const double *const *U, double
         const int i = ids[q];
         const int N = descs[i].order + 1, eb = eb_of[descs[i].nDims * 16 + N];
         hc[q].a = zk::make_args(&descs[i], eb);
-        hc[q].a.trace_sel = (k.op == Op::ExtrapPartner) ? 1 : 0;
         hc[q].U = U[i];
-        hc[q].out = (k.op == Op::Div || k.op == Op::OneSided || k.op == Op::FaceCorr) ? divF[i] : nullptr;
+        if (k.op == Op::BothSidesFromTrace || k.op == Op::FaceCorrBoth) hc[q].a.Ftr = descs[i].Gtr;
+        hc[q].out = (k.op == Op::Extrap) ? nullptr : divF[i];
         hc[q].N = N;
         hc[q].D = descs[i].nDims;
         hs[q] = blocks;

@@ -908,12 +908,6 @@ __global__ __launch_bounds__((Shape<D, N>::kThreads)) void k_gradient(const doub
   gradient_block<D, N>(U, dU_out, a, xcd_block(blockIdx.x, gridDim.x));
 }
 
-template <int D, int N>
-__global__ __launch_bounds__((Shape<D, N>::kThreads)) void k_gradient_multi(const MultiCase *__restrict__ cs, const long *__restrict__ starts, int nc) {
-  const int c = find_case(starts, nc, blockIdx.x);
-  gradient_block<D, N>(cs[c].U, nullptr, cs[c].a, (long)blockIdx.x - starts[c]);
-}
-
 // ---------------------------------------------------------------- kernel 3: divergence
 // compute_F + compute_divF_spts + compute_common_F + compute_divF_fpts.
 // Phases (viscous): U -> LDS | Ucomm -> lC | gradient -> lG | common flux -> lC |
@@ -1186,10 +1180,10 @@ void k_divergence_w64(const double *U, double *__restrict__ divF, KArgs a) {
   divergence_block<D, N, VISC, BM, FC, SELF>(U, divF, a, xcd_block(blockIdx.x, gridDim.x));
 }
 
-template <int D, int N, bool VISC, int BM, int FC>
+template <int D, int N, int FC>
 __global__ __launch_bounds__((Shape<D, N>::kThreads)) void k_divergence_multi(const MultiCase *__restrict__ cs, const long *__restrict__ starts, int nc) {
   const int c = find_case(starts, nc, blockIdx.x);
-  divergence_block<D, N, VISC, BM, FC, !VISC>(cs[c].U, cs[c].out, cs[c].a, (long)blockIdx.x - starts[c]);
+  divergence_block<D, N, false, 0, FC, true>(cs[c].U, cs[c].out, cs[c].a, (long)blockIdx.x - starts[c]);
 }
 
 // ---------------------------------------------------------------- one-sided LDG path
@@ -1202,8 +1196,14 @@ __global__ __launch_bounds__((Shape<D, N>::kThreads)) void k_divergence_multi(co
 // point is extrapolated from the partner's U inside the kernel.  A residual is then
 //   k_visc_onesided (gradient, volume flux divergence, owned common fluxes)
 //   -> k_face_correction (oppDiv_fpts Fcomm, both sides).
+// Any other beta (BM 0) runs through the same two kernels: each side's viscous flux enters
+// the common flux with its own weight, so each side writes its share of the flux at every
+// flux point (5 values where a gradient trace is 15) and k_face_correction adds the two.
+// The three launches it replaces (trace, gradient and its traces, divergence with the
+// gradient and both sides' fluxes formed again) took 84 us per residual of 21x23x19 hexes
+// p=2 and 1.94 ms of 48^2 x 49 hexes p=3.
 
-// Register budget: three waves per SIMD for hex p=3.  The kernel's LDS admits 15 waves per CU,
+// Register budget: three waves per SIMD for hex p=3 and 4.  At p=3 the kernel's LDS admits 15 waves per CU,
 // but 3.2 per SIMD are in flight on average, with the LDS pipe 70% and the VALU 54% busy
 // (64^3, rocprofv3), so a fourth wave buys nothing: held to 128 VGPRs the Roe kernel spills
 // 10 of them (0.37 GB written and read back per residual; 64^3 residual 1627 us), at 148 it
@@ -1211,7 +1211,7 @@ __global__ __launch_bounds__((Shape<D, N>::kThreads)) void k_divergence_multi(co
 // allocation.
 template <int D, int N>
 struct OneSidedWaves {
-  static constexpr int value = (D == 3 && N == 4) ? 3 : 1;
+  static constexpr int value = (D == 3 && (N == 4 || N == 5)) ? 3 : 1;
 };
 
 // SELF: extrapolate the partner traces this element needs from the partner's U (no trace
@@ -1224,7 +1224,7 @@ __device__ __forceinline__ void visc_onesided_block(const double *__restrict__ U
                                                     const KArgs &a, long bid) {
   using S = Shape<D, N>;
   constexpr int nS = S::nS, nF = S::nF, V = S::V;
-  constexpr int owner = (BM == 1) ? 0 : 1;  // slot whose gradient enters the common flux
+  constexpr int owner = (BM == 2) ? 1 : 0;  // slot that forms the convective flux (and, beta = +-1/2, whose gradient enters)
   // one LDS region per element holds the common solution, then (after a barrier) the
   // gradient, then the transformed flux
   constexpr int W = (V * nF > D * V * nS) ? V * nF : D * V * nS;
@@ -1253,7 +1253,59 @@ __device__ __forceinline__ void visc_onesided_block(const double *__restrict__ U
   const int cnt = __popc(mask) * S::nFF;
   double *c = lW + el * W;
   double cp[V];
-  if (t < cnt && valid) {
+  // general beta: the items are all flux points, the owned ones first, and the partner's
+  // trace is needed at each (nothing is parked: with SELF = false partners read every entry
+  // of Utr; the few owned items beyond the first nS fetch it again in the face phase)
+  auto item_fpt = [&](int k) {
+    return (BM == 0 && k >= cnt) ? list_fpt<D, N>(unowned, k - cnt) : list_fpt<D, N>(owned, k);
+  };
+  auto partner = [&](int f, double *x) {
+    long ep; int sl, fp;
+    unpack_nbr<D, N>(a.nbr[e * nF + f], ep, sl, fp);
+    if constexpr (self) {
+      partner_trace<D, N>(U, a.ops, ep, fp, x);
+    } else {
+#pragma unroll
+      for (int v = 0; v < V; v++) x[v] = a.Utr[(ep * V + v) * nF + fp];
+    }
+  };
+  if constexpr (BM == 0) {
+    unsigned nb[S::FPT];
+#pragma unroll
+    for (int k = 0; k < S::FPT; k++) {
+      const int i = t + k * nS;
+      nb[k] = (valid && i < nF) ? a.nbr[e * nF + item_fpt(i)] : 0u;
+    }
+    // the staged block has arrived with the entries (loads return in order): its registers
+    // are free for the lines
+    stage_U_store<D, N>(U, a, lops, lU, e0, neb, V * nS, sr);
+    PartnerLine<D, N> pl[self ? S::FPT : 1];
+    double x[S::FPT][V];
+#pragma unroll
+    for (int k = 0; k < S::FPT; k++) {
+      if (!valid || t + k * nS >= nF) continue;
+      long ep; int sl, fp;
+      unpack_nbr<D, N>(nb[k], ep, sl, fp);
+      if constexpr (self) {
+        partner_line_load<D, N>(U, a.ops, ep, fp, pl[k]);
+      } else {
+#pragma unroll
+        for (int v = 0; v < V; v++) x[k][v] = a.Utr[(ep * V + v) * nF + fp];
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < S::FPT; k++) {
+      const int i = t + k * nS;
+      if (!valid || i >= nF) continue;
+      if constexpr (self) partner_line_reduce<D, N>(pl[k], x[k]);
+      const int f = item_fpt(i);
+#pragma unroll
+      for (int v = 0; v < V; v++) c[v * nF + f] = x[k][v];
+    }
+#pragma unroll
+    for (int v = 0; v < V; v++) cp[v] = x[0][v];
+  }
+  if (BM != 0 && t < cnt && valid) {
     const int f = list_fpt<D, N>(owned, t);
     long ep; int sl, fp;
     unpack_nbr<D, N>(a.nbr[e * nF + f], ep, sl, fp);
@@ -1269,29 +1321,37 @@ __device__ __forceinline__ void visc_onesided_block(const double *__restrict__ U
     for (int v = 0; v < V; v++) c[v * nF + f] = cp[v];
   }
 #pragma unroll 1
-  for (int k = t + nS; k < cnt; k += nS) {
+  for (int k = t + nS; BM != 0 && k < cnt; k += nS) {
     const int f = list_fpt<D, N>(owned, k);
-    long ep; int sl, fp;
-    unpack_nbr<D, N>(a.nbr[e * nF + f], ep, sl, fp);
     double x[V];
-    if constexpr (self) {
-      partner_trace<D, N>(U, a.ops, ep, fp, x);
-    } else {
-#pragma unroll
-      for (int v = 0; v < V; v++) x[v] = a.Utr[(ep * V + v) * nF + fp];
-    }
+    partner(f, x);
 #pragma unroll
     for (int v = 0; v < V; v++) {
       c[v * nF + f] = x[v];
       a.Utr[(e * V + v) * nF + f] = x[v];
     }
   }
-  stage_U_store<D, N>(U, a, lops, lU, e0, neb, V * nS, sr);
+  if constexpr (BM != 0) stage_U_store<D, N>(U, a, lops, lU, e0, neb, V * nS, sr);
   __syncthreads();
   const double *u = lU + el * V * nS;
   double *g_l = lW + el * W;
-  // common solution (= the non-owner side's state): this element's own trace elsewhere
-  if (valid) {
+  // common solution: beta = +-1/2 the non-owner side's state, so this element's own trace
+  // where the partner owns the face; else both sides' traces mixed
+  if (BM == 0 && valid) {
+    for (int k = t; k < nF; k += nS) {
+      const int f = item_fpt(k);
+      int dim, side, base, str;
+      fpt_info<D, N>(f, dim, side, base, str);
+      const double *lE = tab_lE<N>(lops, side);
+#pragma unroll
+      for (int v = 0; v < V; v++) {
+        const double own = line_extrap<N>(lE, u + v * nS, base, str), par = c[v * nF + f];
+        const double l = (k < cnt) ? own : par, r = (k < cnt) ? par : own;
+        c[v * nF + f] = 0.5 * (l + r) - a.ldg_b * (l - r);
+      }
+    }
+  }
+  if (BM != 0 && valid) {
     const int rest = nF - cnt;
 #pragma unroll 1
     for (int k = t; k < rest; k += nS) {
@@ -1320,11 +1380,13 @@ __device__ __forceinline__ void visc_onesided_block(const double *__restrict__ U
     }
   }
   __syncthreads();
-  // common normal flux (unscaled) at the owned flux points -> Ftr
+  // common normal flux (unscaled) at the owned flux points -> Ftr; general beta: this side's
+  // share of it at every flux point (the convective flux and the penalty at owned ones, this
+  // side's viscous flux with its weight at all)
   if (valid) {
 #pragma unroll 1
-    for (int k = t; k < cnt; k += nS) {
-      const int f = list_fpt<D, N>(owned, k);  // face-major: neighbouring lanes, neighbouring points
+    for (int k = t; k < (BM == 0 ? nF : cnt); k += nS) {
+      const int f = item_fpt(k);  // face-major: neighbouring lanes, neighbouring points
       int dim, side, base, str;
       fpt_info<D, N>(f, dim, side, base, str);
       const double *lE = tab_lE<N>(lops, side);
@@ -1335,20 +1397,31 @@ __device__ __forceinline__ void visc_onesided_block(const double *__restrict__ U
       double Uo[V], Up[V];
 #pragma unroll
       for (int v = 0; v < V; v++) Uo[v] = line_extrap<N>(lE, u + v * nS, base, str);
-#pragma unroll
-      for (int v = 0; v < V; v++) Up[v] = (k == t) ? cp[v] : a.Utr[(e * V + v) * nF + f];
       // the convective flux and the LDG penalty first, so that their temporaries and the
       // partner's state are dead before the gradient's lines are gathered (Roe in the other
       // order needs ~350 registers)
       double Fo[V], G[V];
-      if (owner == 0) {
-        conv_common_flux<D, FC>(Uo, Up, n, a, Fo);
 #pragma unroll
-        for (int v = 0; v < V; v++) Fo[v] += a.ldg_tau * (Uo[v] - Up[v]);
-      } else {
-        conv_common_flux<D, FC>(Up, Uo, n, a, Fo);
+      for (int v = 0; v < V; v++) Fo[v] = 0.0;
+      if (BM != 0 || k < cnt) {
+        if (k == t) {
 #pragma unroll
-        for (int v = 0; v < V; v++) Fo[v] += a.ldg_tau * (Up[v] - Uo[v]);
+          for (int v = 0; v < V; v++) Up[v] = cp[v];
+        } else if (BM == 0) {
+          partner(f, Up);
+        } else {
+#pragma unroll
+          for (int v = 0; v < V; v++) Up[v] = a.Utr[(e * V + v) * nF + f];
+        }
+        if (owner == 0) {
+          conv_common_flux<D, FC>(Uo, Up, n, a, Fo);
+#pragma unroll
+          for (int v = 0; v < V; v++) Fo[v] += a.ldg_tau * (Uo[v] - Up[v]);
+        } else {
+          conv_common_flux<D, FC>(Up, Uo, n, a, Fo);
+#pragma unroll
+          for (int v = 0; v < V; v++) Fo[v] += a.ldg_tau * (Up[v] - Uo[v]);
+        }
       }
       asm volatile("" ::: "memory");
       // one variable's line at a time (a compiler barrier after each): 128 VGPRs instead of
@@ -1360,9 +1433,10 @@ __device__ __forceinline__ void visc_onesided_block(const double *__restrict__ U
           asm volatile("" : "+v"(dUj[v]) : : "memory");  // formed here, before the next line is loaded
         }
       }, n, a, G);
-      // the owner's side alone, with weight 1/2 + |beta| = 1
+      // this side's weight 1/2 +- beta: the owner's alone, 1, with beta = +-1/2
+      const double wt = (BM == 0) ? ((k < cnt) ? 0.5 + a.ldg_b : 0.5 - a.ldg_b) : 1.0;
 #pragma unroll
-      for (int v = 0; v < V; v++) Fo[v] += G[v];
+      for (int v = 0; v < V; v++) Fo[v] += wt * G[v];
 #pragma unroll
       for (int v = 0; v < V; v++) __builtin_nontemporal_store(Fo[v], &a.Ftr[(e * V + v) * nF + f]);
     }
@@ -1439,7 +1513,7 @@ template <int D, int N, int BM, int FC>
 __global__ __launch_bounds__((Shape<D, N>::kThreads)) __attribute__((amdgpu_waves_per_eu(OneSidedWaves<D, N>::value)))
 void k_visc_onesided_multi(const MultiCase *__restrict__ cs, const long *__restrict__ starts, int nc) {
   const int c = find_case(starts, nc, blockIdx.x);
-  visc_onesided_block<D, N, BM, FC, true>(cs[c].U, cs[c].out, cs[c].a, (long)blockIdx.x - starts[c]);
+  visc_onesided_block<D, N, BM, FC, BM != 0>(cs[c].U, cs[c].out, cs[c].a, (long)blockIdx.x - starts[c]);
 }
 
 
@@ -1449,7 +1523,7 @@ template <int D, int N, int BM>
 __device__ __forceinline__ void face_correction_block(double *__restrict__ divF, const KArgs &a, long bid) {
   using S = Shape<D, N>;
   constexpr int nS = S::nS, nF = S::nF, V = S::V;
-  constexpr int owner = (BM == 1) ? 0 : 1;
+  constexpr int owner = (BM == 2) ? 1 : 0;
   // per-element LDS block: the common fluxes (V * nF), then the new state (V * nS) when the
   // RK update writes the next trace
   constexpr int W = V * (nF > nS ? nF : nS);
@@ -1473,9 +1547,15 @@ __device__ __forceinline__ void face_correction_block(double *__restrict__ divF,
       long ep; int sl, fp;
       unpack_nbr<D, N>(a.nbr[e * nF + f], ep, sl, fp);
       const double dAs = a.fgeo[(e * (D + 1) + D) * nF + f];
-      const double *src = (sl == owner) ? a.Ftr + e * V * nF + f : a.Ftr + ep * V * nF + fp;
+      if constexpr (BM == 0) {  // both sides' shares
+        const double *so = a.Ftr + e * V * nF + f, *sp = a.Ftr + ep * V * nF + fp;
 #pragma unroll
-      for (int v = 0; v < V; v++) c[v * nF + f] = src[v * nF] * dAs;
+        for (int v = 0; v < V; v++) c[v * nF + f] = (so[v * nF] + sp[v * nF]) * dAs;
+      } else {
+        const double *src = (sl == owner) ? a.Ftr + e * V * nF + f : a.Ftr + ep * V * nF + fp;
+#pragma unroll
+        for (int v = 0; v < V; v++) c[v * nF + f] = src[v * nF] * dAs;
+      }
     }
   }
   __syncthreads();
@@ -1506,8 +1586,8 @@ __device__ __forceinline__ void face_correction_block(double *__restrict__ divF,
     for (int v = 0; v < V; v++) res[v] = acc[v];
     rk_epilogue<D>(a, e, t, nS, acc, unew);
   }
-  // the new state's partner-owned trace for the next stage
-  if (a.rk.mode == 1 && a.rk.trace) rk_trace<D, N>(a, lops, c, e, t, valid, unew, owner);
+  // the new state's trace for the next stage: at partner-owned points, or (general beta) all
+  if (a.rk.mode == 1 && a.rk.trace) rk_trace<D, N>(a, lops, c, e, t, valid, unew, BM == 0 ? -1 : owner);
   // p-multigrid transfers (the common fluxes in c are consumed; U comes from pmgU)
   if (a.rk.pmgRc || a.rk.pmgUf) pmg_epilogue<D, N>(a, lops, nullptr, c, e, t, valid, res, unew);
 }
@@ -1602,6 +1682,7 @@ inline KArgs make_args(const zfr_ele_desc_t *d, int EB) {
 
 enum class Op {
   Extrap, ExtrapPartner, Grad, Div, OneSided, OneSidedFromTrace, FaceCorr,
+  BothSides, BothSidesFromTrace, FaceCorrBoth,  // the one-sided pair's general-beta form
   AdjPrep, AdjMain, AdjGather,  // reverse mode (Euler, LDG beta = +-1/2; AdjPrep and AdjGather also general beta)
   AdjFace, AdjMainGen           // reverse mode, general LDG beta
 };
@@ -1628,9 +1709,12 @@ size_t lds_per_element(Op op, bool viscous) {
     case Op::Div: per_ele = kUC + kG; break;
     case Op::OneSided:
     case Op::OneSidedFromTrace:
-      per_ele = (size_t)S::V * S::nS + (S::V * S::nF > (int)kG ? S::V * S::nF : kG) + 1;
+    case Op::BothSides:
+    case Op::BothSidesFromTrace:
+      per_ele = (size_t)S::V * S::nS + (S::V * S::nF > (int)kG ? S::V * S::nF : kG);
       break;
-    case Op::FaceCorr: per_ele = (size_t)S::V * (S::nF > S::nS ? S::nF : S::nS); break;
+    case Op::FaceCorr:
+    case Op::FaceCorrBoth: per_ele = (size_t)S::V * (S::nF > S::nS ? S::nF : S::nS); break;
     case Op::AdjPrep: per_ele = (size_t)S::V * S::nS; break;
     case Op::AdjMain:
       per_ele = viscous ? (size_t)AdjLds<D, N, true>::per_ele : (size_t)AdjLds<D, N, false>::per_ele;

@@ -73,14 +73,17 @@ int launch(Op op, const zfr_ele_desc_t *d, const double *U, double *out, hipStre
   if ((op == Op::OneSided || op == Op::OneSidedFromTrace || op == Op::FaceCorr) && d->ldg_b != 0.5 &&
       d->ldg_b != -0.5)
     return zfr::fail("one-sided LDG kernels need ldg_b = +-0.5");
-  const bool phased = op == Op::OneSided || op == Op::OneSidedFromTrace || op == Op::Div || op == Op::AdjMain ||
-                      op == Op::AdjMainGen;
+  if ((op == Op::BothSides || op == Op::BothSidesFromTrace || op == Op::FaceCorrBoth) && !general)
+    return zfr::fail("both-sides LDG kernels need a viscous descriptor with ldg_b != +-0.5");
+  const bool phased = op == Op::OneSided || op == Op::OneSidedFromTrace || op == Op::BothSides ||
+                      op == Op::BothSidesFromTrace || op == Op::Div || op == Op::AdjMain || op == Op::AdjMainGen;
   const int EB = eles_per_block(d, S::defaultEB(), S::NOPS_PAD, per_ele, !g_persist, phased);
   if (sizeof(double) * (S::NOPS_PAD + EB * per_ele) > max_lds<D, N>())
     return zfr::fail("kernel launch: one element needs more LDS than a workgroup may use (order too high)");
   KArgs a = make_args(d, EB);
   if (j.rk) {
-    if (op != Op::Div && op != Op::FaceCorr) return zfr::fail("kernel launch: RK fusion is for the last kernel only");
+    if (op != Op::Div && op != Op::FaceCorr && op != Op::FaceCorrBoth)
+      return zfr::fail("kernel launch: RK fusion is for the last kernel only");
     a.rk = *j.rk;
   }
   const dim3 grid((unsigned)((d->nEles + EB - 1) / EB)), block((unsigned)(EB * S::nS));
@@ -122,10 +125,22 @@ int launch(Op op, const zfr_ele_desc_t *d, const double *U, double *out, hipStre
         if (d->fconv_type == 2) { if (d->ldg_b == 0.5) ZK_OS2(k_visc_onesided, 1, 1); else ZK_OS2(k_visc_onesided, 2, 1); }
         else { if (d->ldg_b == 0.5) ZK_OS2(k_visc_onesided, 1, 0); else ZK_OS2(k_visc_onesided, 2, 0); }
       }
+      break;
+    }
+    case Op::BothSides:
+    case Op::BothSidesFromTrace: {
+      const bool self = op == Op::BothSides;
+#define ZK_BS(K_, F_) do { if (self) ZK_OS(K_, 0, F_, true); else ZK_OS(K_, 0, F_, false); } while (0)
+      if (block.x <= 64) { if (d->fconv_type == 2) ZK_BS(k_visc_onesided_w64, 1); else ZK_BS(k_visc_onesided_w64, 0); }
+      else { if (d->fconv_type == 2) ZK_BS(k_visc_onesided, 1); else ZK_BS(k_visc_onesided, 0); }
+#undef ZK_BS
 #undef ZK_OS2
 #undef ZK_OS
       break;
     }
+    case Op::FaceCorrBoth:
+      hipLaunchKernelGGL((k_face_correction<D, N, 0>), grid, block, lds, st, out, a);
+      break;
     case Op::FaceCorr:
       if (d->ldg_b == 0.5) hipLaunchKernelGGL((k_face_correction<D, N, 1>), grid, block, lds, st, out, a);
       else hipLaunchKernelGGL((k_face_correction<D, N, 2>), grid, block, lds, st, out, a);
@@ -168,22 +183,21 @@ void launch_multi(const MultiGroup &g, hipStream_t st) {
     case Op::ExtrapPartner:
       hipLaunchKernelGGL((k_extrapolate_multi<D, N>), grid, block, g.lds, st, c, s0, g.nc);
       break;
-    case Op::Grad:
-      hipLaunchKernelGGL((k_gradient_multi<D, N>), grid, block, g.lds, st, c, s0, g.nc);
-      break;
-    case Op::Div:
-#define ZK_DIV(V_, B_, F_) hipLaunchKernelGGL((k_divergence_multi<D, N, V_, B_, F_>), grid, block, g.lds, st, c, s0, g.nc)
-      if (!g.visc) { if (g.fc) ZK_DIV(false, 0, 1); else ZK_DIV(false, 0, 0); }
-      else if (g.bm == 1) { if (g.fc) ZK_DIV(true, 1, 1); else ZK_DIV(true, 1, 0); }
-      else if (g.bm == 2) { if (g.fc) ZK_DIV(true, 2, 1); else ZK_DIV(true, 2, 0); }
-      else { if (g.fc) ZK_DIV(true, 0, 1); else ZK_DIV(true, 0, 0); }
-#undef ZK_DIV
+    case Op::Div:  // Euler
+      if (g.fc) hipLaunchKernelGGL((k_divergence_multi<D, N, 1>), grid, block, g.lds, st, c, s0, g.nc);
+      else hipLaunchKernelGGL((k_divergence_multi<D, N, 0>), grid, block, g.lds, st, c, s0, g.nc);
       break;
     case Op::OneSided:
 #define ZK_OSM(B_, F_) hipLaunchKernelGGL((k_visc_onesided_multi<D, N, B_, F_>), grid, block, g.lds, st, c, s0, g.nc)
       if (g.bm == 1) { if (g.fc) ZK_OSM(1, 1); else ZK_OSM(1, 0); }
       else { if (g.fc) ZK_OSM(2, 1); else ZK_OSM(2, 0); }
+      break;
+    case Op::BothSidesFromTrace:
+      if (g.fc) ZK_OSM(0, 1); else ZK_OSM(0, 0);
 #undef ZK_OSM
+      break;
+    case Op::FaceCorrBoth:
+      hipLaunchKernelGGL((k_face_correction_multi<D, N, 0>), grid, block, g.lds, st, c, s0, g.nc);
       break;
     case Op::FaceCorr:
       if (g.bm == 1) hipLaunchKernelGGL((k_face_correction_multi<D, N, 1>), grid, block, g.lds, st, c, s0, g.nc);

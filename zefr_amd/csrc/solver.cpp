@@ -348,8 +348,9 @@ void FRSolver::setup_device() {
   el.divF_d.alloc((size_t)input->nStages * st * sizeof(double));
   hip_or_throw(hipMemset(el.divF_d.p, 0, el.divF_d.bytes), "hipMemset");
   el.Utr_d.alloc((size_t)E * V * nF * sizeof(double));
-  if (!onesided() && input->nStages > 1) el.Utr2_d.alloc((size_t)E * V * nF * sizeof(double));
+  if (!input->viscous && input->nStages > 1) el.Utr2_d.alloc((size_t)E * V * nF * sizeof(double));
   if (onesided()) el.Ftr_d.alloc((size_t)E * V * nF * sizeof(double));
+  // general beta: the common-flux shares of a residual, the gradient traces of its VJP
   else if (input->viscous) el.Gtr_d.alloc((size_t)E * D * V * nF * sizeof(double));
   norm_work_d.alloc(1024 * 8 * sizeof(double));
   norm_out_d.alloc(8 * sizeof(double));
@@ -368,19 +369,36 @@ bool FRSolver::onesided() const {
 }
 
 // compute_residual (src/solver.cpp:1494-1645) and its split (:1647-1840):
-//   start  = U traces (extrapolate_U);
-//   mid    = one-sided LDG: gradient, volume divergence and owned common fluxes;
-//            general LDG beta: gradient and its traces;
-//   finish = one-sided LDG: face correction of divF;
-//            otherwise: common flux + full divergence.
+//   start  = nothing on the device (the kernels extrapolate the partner traces themselves);
+//   mid    = viscous: gradient, volume divergence and each face's common flux (beta = +-1/2:
+//            by its owner; other beta: each side's share);
+//   finish = viscous: face correction of divF; Euler: common flux + full divergence.
 const double *FRSolver::cur_state() const { return state_in ? state_in : eles->U_spts_d.as<double>(); }
 
 void FRSolver::compute_residual_start(unsigned, int color) {
   need_device(*this);
   if (color > -1) raise("multi-colour (MCGS) residuals are not supported");
-  const auto d = eles->desc(*input, 0);
-  // the one-sided and the Euler kernels extrapolate the partner traces they need themselves
-  if (input->viscous && !onesided()) status_or_throw(zfr_extrapolate(&d, cur_state(), stream));
+}
+
+// The first viscous launch; traced: the partner traces are in d.Utr (RK stages 1..)
+void FRSolver::viscous_flux(const zfr_ele_desc_t &d, const double *U, double *divF, bool traced, hipStream_t st) {
+  if (!onesided()) {
+    auto g = d;
+    g.Ftr = g.Gtr;
+    status_or_throw(zfr_both_sides_flux(&g, U, divF, traced, st));
+  } else if (traced) status_or_throw(zfr_gradient_flux_traced(&d, U, divF, st));
+  else status_or_throw(zfr_gradient_flux(&d, U, divF, st));
+}
+
+// The last launch of a residual, with an epilogue or without.
+void FRSolver::last_launch(const zfr_ele_desc_t &d, const double *U, double *divF, const zfr_rk_args_t *rk,
+                           hipStream_t st) {
+  if (input->viscous && !onesided()) {
+    auto g = d;
+    g.Ftr = g.Gtr;
+    status_or_throw(zfr_both_sides_correction(&g, divF, rk, st));
+  } else if (input->viscous) status_or_throw(rk ? zfr_face_correction_rk(&d, divF, rk, st) : zfr_face_correction(&d, divF, st));
+  else status_or_throw(rk ? zfr_divergence_rk(&d, U, divF, rk, st) : zfr_divergence(&d, U, divF, st));
 }
 
 void FRSolver::compute_residual_mid(unsigned stage, int) {
@@ -388,23 +406,16 @@ void FRSolver::compute_residual_mid(unsigned stage, int) {
   if (stage >= input->nStages) raise("stage out of range");
   auto d = eles->desc(*input, 1);
   if (trace_in) d.Utr = trace_in;
-  if (onesided()) {
-    double *divF = eles->divF_d.as<double>() + (size_t)stage * eles->state_size();
-    // with trace_in (RK stages 1..), the previous stage's update has written the traces
-    if (trace_in) status_or_throw(zfr_gradient_flux_traced(&d, cur_state(), divF, stream));
-    else status_or_throw(zfr_gradient_flux(&d, cur_state(), divF, stream));
-  } else {
-    status_or_throw(zfr_gradient(&d, cur_state(), nullptr, stream));
-  }
+  // with trace_in (RK stages 1..), the previous stage's update has written the traces
+  viscous_flux(d, cur_state(), eles->divF_d.as<double>() + (size_t)stage * eles->state_size(), trace_in != nullptr,
+               stream);
 }
 
 void FRSolver::compute_residual_finish(unsigned stage, int) {
   if (stage >= input->nStages) raise("stage out of range");
   auto d = eles->desc(*input, 2);
   if (trace_in) d.Utr = trace_in;
-  double *divF = eles->divF_d.as<double>() + (size_t)stage * eles->state_size();
-  if (onesided()) status_or_throw(zfr_face_correction(&d, divF, stream));
-  else status_or_throw(zfr_divergence(&d, cur_state(), divF, stream));
+  last_launch(d, cur_state(), eles->divF_d.as<double>() + (size_t)stage * eles->state_size(), nullptr, stream);
 }
 
 void FRSolver::compute_residual(unsigned stage, int color) {
@@ -416,17 +427,8 @@ void FRSolver::compute_residual(unsigned stage, int color) {
 
 void FRSolver::residual_at(const double *U, double *divF, hipStream_t st) {
   need_device(*this);
-  const auto d0 = eles->desc(*input, 0), d1 = eles->desc(*input, 1), d2 = eles->desc(*input, 2);
-  if (onesided()) {
-    status_or_throw(zfr_gradient_flux(&d1, U, divF, st));
-    status_or_throw(zfr_face_correction(&d2, divF, st));
-  } else {
-    if (input->viscous) {
-      status_or_throw(zfr_extrapolate(&d0, U, st));
-      status_or_throw(zfr_gradient(&d1, U, nullptr, st));
-    }
-    status_or_throw(zfr_divergence(&d2, U, divF, st));  // Euler: extrapolates the partner traces itself
-  }
+  if (input->viscous) viscous_flux(eles->desc(*input, 1), U, divF, false, st);
+  last_launch(eles->desc(*input, 2), U, divF, nullptr, st);
 }
 
 void FRSolver::residual_vjp(const double *U, const double *w, double *v, hipStream_t st) {
@@ -509,8 +511,7 @@ void FRSolver::finish_with_rk(int stage, double *trace_out, bool split) {
     }
   }
   double *divF = eles->divF_d.as<double>() + (size_t)stage * st;
-  if (onesided()) status_or_throw(zfr_face_correction_rk(&d, divF, &r, stream));
-  else status_or_throw(zfr_divergence_rk(&d, cur_state(), divF, &r, stream));
+  last_launch(d, cur_state(), divF, &r, stream);
 }
 
 // One RK step.  Unfused: U_ini = U, then per stage a residual and an update kernel.
@@ -519,11 +520,10 @@ void FRSolver::finish_with_rk(int stage, double *trace_out, bool split) {
 // 1.. update U_ini_d in place; the final combination writes U_spts_d and stores the
 // starting state into U_ini_d (so U_ini_d ends as the unfused step leaves it, and no copy
 // precedes the step).  Each stage update also writes the next stage's trace, so only
-// stage 0 forms it from the state (the extrapolation kernel, or on the one-sided path the
-// gradient_flux kernel itself).  On the one-sided path the writing kernel
-// (face_correction) reads no trace and writes Utr_d in place, and stages 1.. read it
-// (gradient_flux_traced).  On the Euler and general-LDG paths the writing kernel
-// (divergence) reads the partners' traces, so the stages alternate Utr_d and Utr2_d.  An
+// stage 0 forms it from the state (the kernels themselves).  On the viscous paths the
+// writing kernel (the face correction) reads no trace and writes Utr_d in place, and stages
+// 1.. read it.  On the Euler path the writing kernel (divergence) reads the partners'
+// traces, so the stages alternate Utr_d and Utr2_d.  An
 // Euler divergence whose epilogue writes the state it reads (stages 1.., and the final
 // combination, which writes U_ini_d) reads the partners' traces instead of their state;
 // stage 0 of a split step writes only U_ini_d and extrapolates them itself.
@@ -537,17 +537,17 @@ void FRSolver::step_RK_eager() {
     hip_or_throw(hipMemcpyAsync(rk_save, eles->U_spts_d.p, eles->U_spts_d.bytes, hipMemcpyDeviceToDevice, stream),
                  "hipMemcpyAsync");
   double *const tr[2] = {eles->Utr_d.as<double>(),
-                         onesided() ? eles->Utr_d.as<double>() : eles->Utr2_d.as<double>()};
+                         input->viscous ? eles->Utr_d.as<double>() : eles->Utr2_d.as<double>()};
   const bool chain = fuse_rk && ns > 1 && tr[1] != nullptr;
   for (int stage = 0; stage < ns; stage++) {
     if (fuse_rk) {
       trace_in = (chain && stage > 0) ? tr[stage % 2] : nullptr;
       state_in = (split && stage > 0) ? eles->U_ini_d.as<double>() : nullptr;
       try {
-        // the fused divergence reads a trace (viscous, or Euler writing the state it
-        // reads): form it at stage 0, or at every stage without the chain
-        const bool reads_tr = input->viscous || !split || stage > 0;
-        if ((!chain || stage == 0) && !onesided() && reads_tr) {
+        // a fused Euler divergence that writes the state it reads takes its partners' traces:
+        // form them at stage 0, or at every stage without the chain
+        const bool reads_tr = !input->viscous && (!split || stage > 0);
+        if ((!chain || stage == 0) && reads_tr) {
           const auto d0 = eles->desc(*input, 0);
           status_or_throw(zfr_extrapolate(&d0, cur_state(), stream));
         }
@@ -683,8 +683,7 @@ void FRSolver::residual_restrict(const double *source, const double *R, int n_ou
   r.restrict_divF = Rc;
   r.restrict_src = cur_state();
   double *divF = eles->divF_d.as<double>();
-  if (onesided()) status_or_throw(zfr_face_correction_rk(&d, divF, &r, stream));
-  else status_or_throw(zfr_divergence_rk(&d, cur_state(), divF, &r, stream));
+  last_launch(d, cur_state(), divF, &r, stream);
 }
 
 void FRSolver::residual_source(int mode, double *source_out, const double *source) {
@@ -704,8 +703,7 @@ void FRSolver::residual_source(int mode, double *source_out, const double *sourc
   r.mode = mode;
   r.source = source;
   r.source_out = source_out;
-  if (onesided()) status_or_throw(zfr_face_correction_rk(&d, divF, &r, stream));
-  else status_or_throw(zfr_divergence_rk(&d, cur_state(), divF, &r, stream));
+  last_launch(d, cur_state(), divF, &r, stream);
 }
 
 // step_RK_stage (src/solver.cpp:3458-3690)
@@ -792,9 +790,9 @@ int FRSolver::autotune(int reps) {
   // an inviscid residual has no middle launch: phase 1 timed only the gap between two
   // events, so its tile is the divergence launch's
   if (!input->viscous) best_eb[1] = best_eb[2];
-  // one-sided and Euler residuals have no trace launch, so phase 0 timed nothing; its tile
-  // (used by a fused RK step's stage-0 extrapolation) falls back to the solver-wide tile
-  if (!(input->viscous && !onesided())) best_eb[0] = 0;
+  // no residual has a trace launch, so phase 0 timed nothing; its tile (an Euler RK step's
+  // extrapolation without the trace chain) falls back to the solver-wide tile
+  best_eb[0] = 0;
   el.tile = best_eb[1];
   for (int k = 0; k < 3; k++) el.tile_phase[k] = best_eb[k];
   return best_eb[1];
@@ -804,7 +802,7 @@ int FRSolver::autotune(int reps) {
 void FRSolver::time_kernels(int reps, double *ms_out) {
   need_device(*this);
   Elements &el = *eles;
-  const auto d0 = el.desc(*input, 0), d1 = el.desc(*input, 1), d2 = el.desc(*input, 2);
+  const auto d1 = el.desc(*input, 1), d2 = el.desc(*input, 2);
   reps = std::max(reps, 1);
   // one event before each launch and one after the last: residuals run back to back
   std::vector<hipEvent_t> ev(3 * reps + 1);
@@ -812,13 +810,11 @@ void FRSolver::time_kernels(int reps, double *ms_out) {
   double *U = el.U_spts_d.as<double>(), *divF = el.divF_d.as<double>();
   for (int r = 0; r < reps; r++) {
     hip_or_throw(hipEventRecord(ev[3 * r], stream), "hipEventRecord");
-    if (input->viscous && !onesided()) status_or_throw(zfr_extrapolate(&d0, U, stream));  // else no trace launch
+    // no trace launch (phase 0)
     hip_or_throw(hipEventRecord(ev[3 * r + 1], stream), "hipEventRecord");
-    if (onesided()) status_or_throw(zfr_gradient_flux(&d1, U, divF, stream));
-    else if (input->viscous) status_or_throw(zfr_gradient(&d1, U, nullptr, stream));
+    if (input->viscous) viscous_flux(d1, U, divF, false, stream);
     hip_or_throw(hipEventRecord(ev[3 * r + 2], stream), "hipEventRecord");
-    if (onesided()) status_or_throw(zfr_face_correction(&d2, divF, stream));
-    else status_or_throw(zfr_divergence(&d2, U, divF, stream));
+    last_launch(d2, U, divF, nullptr, stream);
   }
   hip_or_throw(hipEventRecord(ev[3 * reps], stream), "hipEventRecord");
   hip_or_throw(hipEventSynchronize(ev[3 * reps]), "hipEventSynchronize");
