@@ -932,22 +932,41 @@ __device__ __forceinline__ void divergence_block(const double *U, double *__rest
   const int tid = threadIdx.x, el = tid / nS, t = tid - el * nS;
   const long e = e0 + el;
   const bool valid = el < neb;
-  // Euler: everything this thread reads from global memory besides the staged block (the
-  // partner states and face geometry of its flux points, its metric, the RK epilogue's
-  // inputs) is loaded here, before the staging, so that the loads overlap one another
-  // instead of each costing a memory round trip between the phases
+  // Euler: everything this thread reads from global memory is loaded here, ahead of the first
+  // barrier: first all that depends on nothing (the staged block, the partner entries and
+  // face geometry of its flux points, its metric, the RK epilogue's inputs), then the partner
+  // states.  Two dependent round trips; taken flux point by flux point, with the rest behind
+  // them, they were 2 FPT + 1, and on small meshes a launch is little else.  Out-of-range
+  // threads and points load a neighbour's data (in bounds) instead of branching.  (29x31x27
+  // hexes p=2, RK44 step 246 -> 232 us; 128^2 quads p=4, V-cycle 520 -> 495.)
   constexpr int PF = VISC ? 1 : S::FPT;
   double pUs[PF][V], pn[PF][D], pdA[PF], pij[D][D], pdet = 1.0;
   int psl[PF];
   RkPre<D> pre;
-  if (!VISC && valid) {
+  if constexpr (!VISC) {
+    const long ec = valid ? e : e0;
+    StageRegs<D, N> sr;
+    stage_U_load<D, N>(U, a, e0, neb, sr);
+    unsigned nb[PF];
 #pragma unroll
     for (int k = 0; k < PF; k++) {
       const int f = t + k * nS;
-      psl[k] = 0;
-      if (f >= nF) continue;
+      nb[k] = a.nbr[ec * nF + (f < nF ? f : 0)];
+    }
+#pragma unroll
+    for (int k = 0; k < PF; k++) {
+      const int f = t + k * nS;
+      const double *fg = a.fgeo + ec * (D + 1) * nF + (f < nF ? f : 0);
+#pragma unroll
+      for (int d = 0; d < D; d++) pn[k][d] = fg[d * nF];
+      pdA[k] = fg[D * nF];
+    }
+    load_metric<D>(a, ec, t, nS, pij, pdet, false);
+    rk_prefetch<D>(a, ec, t, nS, pre);
+#pragma unroll
+    for (int k = 0; k < PF; k++) {
       long ep; int sl, fp;
-      unpack_nbr<D, N>(a.nbr[e * nF + f], ep, sl, fp);
+      unpack_nbr<D, N>(nb[k], ep, sl, fp);
       psl[k] = sl;
       if constexpr (SELF) {
         partner_trace<D, N>(U, a.ops, ep, fp, pUs[k]);
@@ -955,15 +974,11 @@ __device__ __forceinline__ void divergence_block(const double *U, double *__rest
 #pragma unroll
         for (int v = 0; v < V; v++) pUs[k][v] = a.Utr[(ep * V + v) * nF + fp];
       }
-      const double *fg = a.fgeo + e * (D + 1) * nF + f;
-#pragma unroll
-      for (int d = 0; d < D; d++) pn[k][d] = fg[d * nF];
-      pdA[k] = fg[D * nF];
     }
-    load_metric<D>(a, e, t, nS, pij, pdet, false);
-    rk_prefetch<D>(a, e, t, nS, pre);
+    stage_U_store<D, N>(U, a, lops, lU, e0, neb, V * nS, sr);
+  } else {
+    stage_U<D, N>(U, a, lops, lU, e0, neb, V * nS);
   }
-  stage_U<D, N>(U, a, lops, lU, e0, neb, V * nS);
   __syncthreads();
   const double *u = lU + el * V * nS;
   double *c = lC + el * V * nF;
