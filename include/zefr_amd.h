@@ -405,11 +405,9 @@ int zfr_face_correction_rk(const zfr_ele_desc_t *d, double *divF, const zfr_rk_a
 /* The two launches of a viscous residual with LDG beta other than +-1/2 (both sides' gradients
  * in each common flux, src/faces.cpp:1476-1614), as zfr_gradient_flux and zfr_face_correction
  * are for beta = +-1/2: the first writes the volume part of divF and this side's share of the
- * common flux at every flux point to d->Ftr, the second adds both sides' shares.  The partner
- * traces come from the partners' U, or (traced != 0) from d->Utr at every flux point, as
- * zfr_extrapolate or a fused update's trace_out writes it.  rk: an epilogue as in
- * zfr_face_correction_rk (trace_out takes every flux point and may be d->Utr), or NULL. */
-int zfr_both_sides_flux(const zfr_ele_desc_t *d, const double *U, double *divF, int traced, void *stream);
+ * common flux at every flux point to d->Ftr, the second adds both sides' shares.  rk: an
+ * epilogue as in zfr_face_correction_rk (trace_out takes every flux point), or NULL. */
+int zfr_both_sides_flux(const zfr_ele_desc_t *d, const double *U, double *divF, void *stream);
 int zfr_both_sides_correction(const zfr_ele_desc_t *d, double *divF, const zfr_rk_args_t *rk, void *stream);
 int zfr_divergence_rk(const zfr_ele_desc_t *d, const double *U, double *divF, const zfr_rk_args_t *rk,
                       void *stream);

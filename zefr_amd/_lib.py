@@ -152,7 +152,7 @@ SIGNATURES = {
     "zfr_residual_norm_static": (_I, [C.POINTER(EleDesc), _P, _I, _P, _P]),
     "zfr_residual_vjp": (_I, [C.POINTER(EleDesc), _P, _P, _P, _P, _P, _P]),
     "zfr_face_correction_rk": (_I, [C.POINTER(EleDesc), _P, _P, _P]),
-    "zfr_both_sides_flux": (_I, [C.POINTER(EleDesc), _P, _P, _I, _P]),
+    "zfr_both_sides_flux": (_I, [C.POINTER(EleDesc), _P, _P, _P]),
     "zfr_both_sides_correction": (_I, [C.POINTER(EleDesc), _P, _P, _P]),
     "zfr_divergence_rk": (_I, [C.POINTER(EleDesc), _P, _P, _P, _P]),
     "zfr_stream_copy": (_I, [_P, _P, C.c_long, _P]),

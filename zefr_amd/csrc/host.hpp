@@ -108,7 +108,7 @@ class Elements {
   std::vector<double> metric;                        // [E][D*D+1][nS]: adjugate(d1,d2), detJ
   // device data (element-major)
   DevBuf U_spts_d, U_ini_d, divF_d, dU_spts_d, metric_d, fgeo_d, nbr_d, ops_d, Utr_d, Gtr_d, Ftr_d;
-  DevBuf Utr2_d;  // second trace buffer: fused RK stages on the divergence path alternate with Utr_d
+  DevBuf U_stage_d;  // Euler, several stages: the stage states of a fused step alternate between this and U_ini_d
   std::vector<double> U_host, dU_host;  // host mirrors for get_u_spts / get_du_spts
   int tile = 0;                         // elements per workgroup (0 = kernel default)
 
@@ -168,7 +168,7 @@ class FRSolver {
   void synchronize();
   int autotune(int reps);
   bool onesided() const;  // viscous with LDG beta = +-1/2: one-sided gradient path
-  void viscous_flux(const zfr_ele_desc_t &d, const double *U, double *divF, bool traced, hipStream_t st);
+  void viscous_flux(const zfr_ele_desc_t &d, const double *U, double *divF, hipStream_t st);
   void last_launch(const zfr_ele_desc_t &d, const double *U, double *divF, const zfr_rk_args_t *rk, hipStream_t st);
   void time_kernels(int reps, double *ms_out);
   // The residual of an arbitrary device state U [E][V][nS] into divF (same layout) on the
@@ -228,11 +228,8 @@ class FRSolver {
   // (divF += source).  With fuse_rk the last residual kernel does it; otherwise an axpby.
   void residual_source(int mode, double *source_out, const double *source);
   bool own_stream = true;  // false for p-multigrid levels, which run on the fine stream
-  // The trace buffer the residual phases read, when not Utr_d (fused RK steps on the
-  // divergence path alternate two buffers; see step_RK_eager)
-  double *trace_in = nullptr;
   // The state the residual phases read, when not U_spts_d (stages 1.. of a fused step,
-  // whose stage states live in U_ini_d; see step_RK_eager)
+  // whose stage states live in U_ini_d and U_stage_d; see step_RK_eager)
   const double *state_in = nullptr;
   // PyFR-format solution files (src/solver.cpp:4275-4837): write returns the file name
   std::string write_solution_pyfr(const std::string &prefix);
@@ -242,7 +239,7 @@ class FRSolver {
  private:
   void rk_stage_update(int stage);
   void rk_final_update();
-  void finish_with_rk(int stage, double *trace_out, bool split);
+  void finish_with_rk(int stage, double *stage_out, bool split);
   const double *cur_state() const;
   void step_RK_eager();
   void drop_graph();

@@ -510,14 +510,13 @@ int rk_fused(zk::Op op, const zfr_ele_desc_t *d, const double *U, double *divF, 
 
 extern "C" {
 
-int zfr_both_sides_flux(const zfr_ele_desc_t *d, const double *U, double *divF, int traced, void *stream) {
+int zfr_both_sides_flux(const zfr_ele_desc_t *d, const double *U, double *divF, void *stream) {
   int rc = need_geometry(d);
   if (!rc) rc = need_arg(U, "U");
   if (!rc) rc = need_arg(divF, "divF");
-  if (!rc && traced) rc = need(d->Utr, "Utr");
   if (!rc) rc = need(d->Ftr, "Ftr");
   if (rc) return rc;
-  return zk::dispatch(traced ? zk::Op::BothSidesFromTrace : zk::Op::BothSides, d, U, divF, (hipStream_t)stream);
+  return zk::dispatch(zk::Op::BothSides, d, U, divF, (hipStream_t)stream);
 }
 
 int zfr_both_sides_correction(const zfr_ele_desc_t *d, double *divF, const zfr_rk_args_t *rk, void *stream) {

@@ -1697,7 +1697,8 @@ inline KArgs make_args(const zfr_ele_desc_t *d, int EB) {
 
 enum class Op {
   Extrap, ExtrapPartner, Grad, Div, OneSided, OneSidedFromTrace, FaceCorr,
-  BothSides, BothSidesFromTrace, FaceCorrBoth,  // the one-sided pair's general-beta form
+  BothSides, FaceCorrBoth,  // the one-sided pair's general-beta form
+  BothSidesFromTrace,       // the same after a trace launch (multi-case launches)
   AdjPrep, AdjMain, AdjGather,  // reverse mode (Euler, LDG beta = +-1/2; AdjPrep and AdjGather also general beta)
   AdjFace, AdjMainGen           // reverse mode, general LDG beta
 };

@@ -73,10 +73,10 @@ int launch(Op op, const zfr_ele_desc_t *d, const double *U, double *out, hipStre
   if ((op == Op::OneSided || op == Op::OneSidedFromTrace || op == Op::FaceCorr) && d->ldg_b != 0.5 &&
       d->ldg_b != -0.5)
     return zfr::fail("one-sided LDG kernels need ldg_b = +-0.5");
-  if ((op == Op::BothSides || op == Op::BothSidesFromTrace || op == Op::FaceCorrBoth) && !general)
+  if ((op == Op::BothSides || op == Op::FaceCorrBoth) && !general)
     return zfr::fail("both-sides LDG kernels need a viscous descriptor with ldg_b != +-0.5");
-  const bool phased = op == Op::OneSided || op == Op::OneSidedFromTrace || op == Op::BothSides ||
-                      op == Op::BothSidesFromTrace || op == Op::Div || op == Op::AdjMain || op == Op::AdjMainGen;
+  const bool phased = op == Op::OneSided || op == Op::OneSidedFromTrace || op == Op::BothSides || op == Op::Div ||
+                      op == Op::AdjMain || op == Op::AdjMainGen;
   const int EB = eles_per_block(d, S::defaultEB(), S::NOPS_PAD, per_ele, !g_persist, phased);
   if (sizeof(double) * (S::NOPS_PAD + EB * per_ele) > max_lds<D, N>())
     return zfr::fail("kernel launch: one element needs more LDS than a workgroup may use (order too high)");
@@ -127,13 +127,9 @@ int launch(Op op, const zfr_ele_desc_t *d, const double *U, double *out, hipStre
       }
       break;
     }
-    case Op::BothSides:
-    case Op::BothSidesFromTrace: {
-      const bool self = op == Op::BothSides;
-#define ZK_BS(K_, F_) do { if (self) ZK_OS(K_, 0, F_, true); else ZK_OS(K_, 0, F_, false); } while (0)
-      if (block.x <= 64) { if (d->fconv_type == 2) ZK_BS(k_visc_onesided_w64, 1); else ZK_BS(k_visc_onesided_w64, 0); }
-      else { if (d->fconv_type == 2) ZK_BS(k_visc_onesided, 1); else ZK_BS(k_visc_onesided, 0); }
-#undef ZK_BS
+    case Op::BothSides: {
+      if (block.x <= 64) { if (d->fconv_type == 2) ZK_OS(k_visc_onesided_w64, 0, 1, true); else ZK_OS(k_visc_onesided_w64, 0, 0, true); }
+      else { if (d->fconv_type == 2) ZK_OS(k_visc_onesided, 0, 1, true); else ZK_OS(k_visc_onesided, 0, 0, true); }
 #undef ZK_OS2
 #undef ZK_OS
       break;
@@ -166,6 +162,8 @@ int launch(Op op, const zfr_ele_desc_t *d, const double *U, double *out, hipStre
       else hipLaunchKernelGGL((k_adj_face<D, N, 0>), fgrid, fblock, 0, st, j.Wtr, a);
       break;
     }
+    case Op::BothSidesFromTrace:  // in multi-case launches only
+      return zfr::fail("kernel launch: no launch of its own");
     case Op::AdjMainGen:
       if constexpr (kAdjoint<D, N>) hipLaunchKernelGGL((k_adj_main_gen<D, N>), grid, block, lds, st, U, j.w, j.Xtr, out, a);
       break;

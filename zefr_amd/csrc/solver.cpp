@@ -348,7 +348,7 @@ void FRSolver::setup_device() {
   el.divF_d.alloc((size_t)input->nStages * st * sizeof(double));
   hip_or_throw(hipMemset(el.divF_d.p, 0, el.divF_d.bytes), "hipMemset");
   el.Utr_d.alloc((size_t)E * V * nF * sizeof(double));
-  if (!input->viscous && input->nStages > 1) el.Utr2_d.alloc((size_t)E * V * nF * sizeof(double));
+  if (!input->viscous && input->nStages > 1) el.U_stage_d.alloc(st * sizeof(double));
   if (onesided()) el.Ftr_d.alloc((size_t)E * V * nF * sizeof(double));
   // general beta: the common-flux shares of a residual, the gradient traces of its VJP
   else if (input->viscous) el.Gtr_d.alloc((size_t)E * D * V * nF * sizeof(double));
@@ -380,14 +380,13 @@ void FRSolver::compute_residual_start(unsigned, int color) {
   if (color > -1) raise("multi-colour (MCGS) residuals are not supported");
 }
 
-// The first viscous launch; traced: the partner traces are in d.Utr (RK stages 1..)
-void FRSolver::viscous_flux(const zfr_ele_desc_t &d, const double *U, double *divF, bool traced, hipStream_t st) {
+// The first viscous launch.
+void FRSolver::viscous_flux(const zfr_ele_desc_t &d, const double *U, double *divF, hipStream_t st) {
   if (!onesided()) {
     auto g = d;
     g.Ftr = g.Gtr;
-    status_or_throw(zfr_both_sides_flux(&g, U, divF, traced, st));
-  } else if (traced) status_or_throw(zfr_gradient_flux_traced(&d, U, divF, st));
-  else status_or_throw(zfr_gradient_flux(&d, U, divF, st));
+    status_or_throw(zfr_both_sides_flux(&g, U, divF, st));
+  } else status_or_throw(zfr_gradient_flux(&d, U, divF, st));
 }
 
 // The last launch of a residual, with an epilogue or without.
@@ -404,18 +403,13 @@ void FRSolver::last_launch(const zfr_ele_desc_t &d, const double *U, double *div
 void FRSolver::compute_residual_mid(unsigned stage, int) {
   if (!input->viscous) return;
   if (stage >= input->nStages) raise("stage out of range");
-  auto d = eles->desc(*input, 1);
-  if (trace_in) d.Utr = trace_in;
-  // with trace_in (RK stages 1..), the previous stage's update has written the traces
-  viscous_flux(d, cur_state(), eles->divF_d.as<double>() + (size_t)stage * eles->state_size(), trace_in != nullptr,
+  viscous_flux(eles->desc(*input, 1), cur_state(), eles->divF_d.as<double>() + (size_t)stage * eles->state_size(),
                stream);
 }
 
 void FRSolver::compute_residual_finish(unsigned stage, int) {
   if (stage >= input->nStages) raise("stage out of range");
-  auto d = eles->desc(*input, 2);
-  if (trace_in) d.Utr = trace_in;
-  last_launch(d, cur_state(), eles->divF_d.as<double>() + (size_t)stage * eles->state_size(), nullptr, stream);
+  last_launch(eles->desc(*input, 2), cur_state(), eles->divF_d.as<double>() + (size_t)stage * eles->state_size(), nullptr, stream);
 }
 
 void FRSolver::compute_residual(unsigned stage, int color) {
@@ -427,7 +421,7 @@ void FRSolver::compute_residual(unsigned stage, int color) {
 
 void FRSolver::residual_at(const double *U, double *divF, hipStream_t st) {
   need_device(*this);
-  if (input->viscous) viscous_flux(eles->desc(*input, 1), U, divF, false, st);
+  if (input->viscous) viscous_flux(eles->desc(*input, 1), U, divF, st);
   last_launch(eles->desc(*input, 2), U, divF, nullptr, st);
 }
 
@@ -473,18 +467,16 @@ void FRSolver::rk_final_update() {
                                       beta, ns, input->dt, stream));
 }
 
-// compute_residual_finish with the RK update of this stage done by the same kernel; with
-// trace_out, that kernel also writes the new state's trace there (stage updates only).
+// compute_residual_finish with the RK update of this stage done by the same kernel.
 // split: the step keeps its starting state in U_spts_d until the final combination and
-// its stage states in U_ini_d (see step_RK_eager).
-void FRSolver::finish_with_rk(int stage, double *trace_out, bool split) {
-  auto d = eles->desc(*input, 2);
-  if (trace_in) d.Utr = trace_in;
+// writes this stage's state to stage_out (see step_RK_eager).
+void FRSolver::finish_with_rk(int stage, double *stage_out, bool split) {
+  const auto d = eles->desc(*input, 2);
   const int ns = (int)input->nStages;
   const size_t st = eles->state_size();
   double *const A = eles->U_spts_d.as<double>(), *const I = eles->U_ini_d.as<double>();
   zfr_rk_args_t r{};
-  r.U = (split && stage < ns - 1) ? I : A;
+  r.U = (split && stage < ns - 1) ? stage_out : A;
   r.U_ini = (split || ns == 1) ? A : I;
   r.divF0 = eles->divF_d.as<double>();
   r.stage = stage;
@@ -496,7 +488,6 @@ void FRSolver::finish_with_rk(int stage, double *trace_out, bool split) {
   if (stage < ns - 1) {
     r.mode = 1;
     r.alpha = kRkAlpha[stage];
-    r.trace_out = trace_out;
   } else {
     r.mode = 2;
     for (int s = 0; s < ns; s++) r.beta[s] = (ns > 1) ? kRkBeta[s] : 1.0;
@@ -515,18 +506,21 @@ void FRSolver::finish_with_rk(int stage, double *trace_out, bool split) {
 }
 
 // One RK step.  Unfused: U_ini = U, then per stage a residual and an update kernel.
-// Fused with several stages (split): the starting state stays in U_spts_d, stage 0's
-// residual is formed from it and its update writes the stage state into U_ini_d; stages
-// 1.. update U_ini_d in place; the final combination writes U_spts_d and stores the
-// starting state into U_ini_d (so U_ini_d ends as the unfused step leaves it, and no copy
-// precedes the step).  Each stage update also writes the next stage's trace, so only
-// stage 0 forms it from the state (the kernels themselves).  On the viscous paths the
-// writing kernel (the face correction) reads no trace and writes Utr_d in place, and stages
-// 1.. read it.  On the Euler path the writing kernel (divergence) reads the partners'
-// traces, so the stages alternate Utr_d and Utr2_d.  An
-// Euler divergence whose epilogue writes the state it reads (stages 1.., and the final
-// combination, which writes U_ini_d) reads the partners' traces instead of their state;
-// stage 0 of a split step writes only U_ini_d and extrapolates them itself.
+// Fused with several stages (split): the starting state stays in U_spts_d, the stage states
+// live in other buffers, and the final combination writes U_spts_d and stores the starting
+// state into U_ini_d (so U_ini_d ends as the unfused step leaves it, and no copy precedes
+// the step).
+// Viscous: the writing kernel (the face correction) reads no state, so every stage's state
+// is written to U_ini_d in place.  Euler: the one kernel of a stage reads its partners'
+// states while it writes, so the stages alternate U_stage_d and U_ini_d, the last of them
+// U_stage_d, and no stage writes the buffer it reads.  Either way every stage extrapolates
+// its partners' traces from their states.  When a stage's update also wrote the new state's
+// trace for the next one to read, these bandwidth-bound kernels moved more (Euler hexes
+// p=2: 12.7 KB per element and stage, 4.3 of them traces, at 5.1 TB/s) and gained two
+// barriers.  RK44 step, with traces against without: 29x31x27 hexes p=2 Euler 238 / 191 us,
+// Navier-Stokes 442 / 390; 32^3 hexes p=3 Euler 706 / 643, Navier-Stokes with Roe 1027 /
+// 984; 256^2 quads p=3 Euler 200 / 178; 128^2 quads p=4 Navier-Stokes 172 / 164;
+// 13x11x17 hexes p=5 Euler 163 / 157; V-cycle of 128^2 quads p=4 513 / 468.
 void FRSolver::step_RK_eager() {
   const int ns = (int)input->nStages;
   const bool split = fuse_rk && ns > 1;
@@ -536,29 +530,25 @@ void FRSolver::step_RK_eager() {
   if (rk_save && !split)
     hip_or_throw(hipMemcpyAsync(rk_save, eles->U_spts_d.p, eles->U_spts_d.bytes, hipMemcpyDeviceToDevice, stream),
                  "hipMemcpyAsync");
-  double *const tr[2] = {eles->Utr_d.as<double>(),
-                         input->viscous ? eles->Utr_d.as<double>() : eles->Utr2_d.as<double>()};
-  const bool chain = fuse_rk && ns > 1 && tr[1] != nullptr;
+  const bool two = split && !input->viscous && eles->U_stage_d.p;  // no second buffer: `viscous` was cleared after setup
+  auto stage_buf = [&](int stage) {
+    return (two && (ns - 2 - stage) % 2 == 0) ? eles->U_stage_d.as<double>() : eles->U_ini_d.as<double>();
+  };
   for (int stage = 0; stage < ns; stage++) {
     if (fuse_rk) {
-      trace_in = (chain && stage > 0) ? tr[stage % 2] : nullptr;
-      state_in = (split && stage > 0) ? eles->U_ini_d.as<double>() : nullptr;
+      state_in = (split && stage > 0) ? stage_buf(stage - 1) : nullptr;
       try {
-        // a fused Euler divergence that writes the state it reads takes its partners' traces:
-        // form them at stage 0, or at every stage without the chain
-        const bool reads_tr = !input->viscous && (!split || stage > 0);
-        if ((!chain || stage == 0) && reads_tr) {
+        // an Euler divergence that writes the state it reads takes its partners' traces
+        if (!input->viscous && !two && (!split || stage > 0)) {
           const auto d0 = eles->desc(*input, 0);
           status_or_throw(zfr_extrapolate(&d0, cur_state(), stream));
         }
         compute_residual_mid(stage);
-        finish_with_rk(stage, (chain && stage < ns - 1) ? tr[(stage + 1) % 2] : nullptr, split);
+        finish_with_rk(stage, (split && stage < ns - 1) ? stage_buf(stage) : nullptr, split);
       } catch (...) {
-        trace_in = nullptr;
         state_in = nullptr;
         throw;
       }
-      trace_in = nullptr;
       state_in = nullptr;
     } else {
       compute_residual(stage);
@@ -790,8 +780,8 @@ int FRSolver::autotune(int reps) {
   // an inviscid residual has no middle launch: phase 1 timed only the gap between two
   // events, so its tile is the divergence launch's
   if (!input->viscous) best_eb[1] = best_eb[2];
-  // no residual has a trace launch, so phase 0 timed nothing; its tile (an Euler RK step's
-  // extrapolation without the trace chain) falls back to the solver-wide tile
+  // no residual has a trace launch, so phase 0 timed nothing; its tile (the extrapolation of
+  // a one-stage Euler step) falls back to the solver-wide tile
   best_eb[0] = 0;
   el.tile = best_eb[1];
   for (int k = 0; k < 3; k++) el.tile_phase[k] = best_eb[k];
@@ -812,7 +802,7 @@ void FRSolver::time_kernels(int reps, double *ms_out) {
     hip_or_throw(hipEventRecord(ev[3 * r], stream), "hipEventRecord");
     // no trace launch (phase 0)
     hip_or_throw(hipEventRecord(ev[3 * r + 1], stream), "hipEventRecord");
-    if (input->viscous) viscous_flux(d1, U, divF, false, stream);
+    if (input->viscous) viscous_flux(d1, U, divF, stream);
     hip_or_throw(hipEventRecord(ev[3 * r + 2], stream), "hipEventRecord");
     last_launch(d2, U, divF, nullptr, stream);
   }
