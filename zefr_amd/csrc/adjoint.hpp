@@ -83,9 +83,10 @@ __global__ __launch_bounds__((Shape<D, N>::kThreads)) void k_adj_prep(const doub
 template <int D, int N, bool VISC>
 struct AdjLds {
   using S = Shape<D, N>;
-  static constexpr int R = (S::V * S::nF > D * S::V * S::nS || !VISC) ? S::V * S::nF : D * S::V * S::nS;
-  static constexpr int GB = VISC ? D * S::V * S::nS : S::V * S::nS;
-  static constexpr int per_ele = S::V * S::nS + R + GB;  // doubles
+  static constexpr int U = S::ele(S::V * S::nS);
+  static constexpr int R = S::ele((S::V * S::nF > D * S::V * S::nS || !VISC) ? S::V * S::nF : D * S::V * S::nS);
+  static constexpr int GB = S::ele(VISC ? D * S::V * S::nS : S::V * S::nS);
+  static constexpr int per_ele = U + R + GB;  // doubles
 };
 
 // The partner's trace at this thread's owned flux point f: its neighbour entry, then its
@@ -144,14 +145,14 @@ __device__ __forceinline__ void adj_visc_block(const double *__restrict__ U, con
   const int EB = a.EB;
   double *lops = lds;
   double *lU = lops + S::NOPS_PAD;
-  double *lR = lU + EB * V * nS;
+  double *lR = lU + EB * L::U;
   double *lGB = lR + EB * L::R;
   const long e0 = bid * EB;
   const long neb = min((long)EB, (long)a.E - e0);
   const int tid = threadIdx.x, el = tid / nS, t = tid - el * nS;
   const long e = e0 + el;
   const bool valid = el < neb;
-  double *u = lU + el * V * nS;
+  double *u = lU + el * L::U;
   double *c = lR + el * L::R, *g_l = c, *T = c, *to = c;
   double *gb = lGB + el * L::GB;
   // 0. staging loads of U and w, the owned faces, and the partner's trace at this thread's
@@ -189,7 +190,7 @@ __device__ __forceinline__ void adj_visc_block(const double *__restrict__ U, con
       a.Utr[(e * V + v) * nF + f] = x[v];
     }
   }
-  stage_U_store<D, N>(U, a, lops, lU, e0, neb, V * nS, sr);
+  stage_U_store<D, N>(U, a, lops, lU, e0, neb, L::U, sr);
   if (valid) {
 #pragma unroll
     for (int v = 0; v < V; v++) gb[v * nS + t] = wr[v];
@@ -471,7 +472,7 @@ __device__ __forceinline__ void adj_euler_block(const double *__restrict__ U, co
   const int EB = a.EB;
   double *lops = lds;
   double *lU = lops + S::NOPS_PAD;
-  double *lT = lU + EB * V * nS;
+  double *lT = lU + EB * L::U;
   double *lw = lT + EB * L::R;
   const long e0 = bid * EB;
   const long neb = min((long)EB, (long)a.E - e0);
@@ -490,9 +491,9 @@ __device__ __forceinline__ void adj_euler_block(const double *__restrict__ U, co
   if (valid) load_metric<D>(a, e, t, nS, ij, detJ, false);
   double cp[V];
   if (t < cnt) owned_partner_trace<D, N>(U, a, e, list_fpt<D, N>(owned, t), cp);
-  stage_U_store<D, N>(U, a, lops, lU, e0, neb, V * nS, sr);
-  const double *u = lU + el * V * nS;
-  double *to = lT + el * L::R, *we = lw + el * V * nS;
+  stage_U_store<D, N>(U, a, lops, lU, e0, neb, L::U, sr);
+  const double *u = lU + el * L::U;
+  double *to = lT + el * L::R, *we = lw + el * L::GB;
   if (valid) {
 #pragma unroll
     for (int v = 0; v < V; v++) we[v * nS + t] = wr[v];
@@ -610,7 +611,7 @@ __global__ __launch_bounds__((Shape<D, N>::kThreads)) void k_adj_gather(const do
   const int el = tid / nS, t = tid - el * nS;
   const long e = e0 + el;
   const bool valid = el < neb;
-  double *T = lT + el * V * nF;
+  double *T = lT + el * S::ele(V * nF);
   if (valid) {
 #pragma unroll
     for (int k = 0; k < S::FPT; k++) {
@@ -734,8 +735,10 @@ __global__ __launch_bounds__(kMaxThreads) void k_adj_face(const double *__restri
 template <int D, int N>
 struct AdjGenLds {
   using S = Shape<D, N>;
-  static constexpr int R = (2 * D * S::V * S::nFF > S::V * S::nF) ? 2 * D * S::V * S::nFF : S::V * S::nF;
-  static constexpr int per_ele = S::V * S::nS + R + D * S::V * S::nS;  // doubles
+  static constexpr int U = S::ele(S::V * S::nS);
+  static constexpr int R = S::ele((2 * D * S::V * S::nFF > S::V * S::nF) ? 2 * D * S::V * S::nFF : S::V * S::nF);
+  static constexpr int GB = S::ele(D * S::V * S::nS);
+  static constexpr int per_ele = U + R + GB;  // doubles
 };
 
 template <int D, int N>
@@ -749,23 +752,23 @@ __device__ __forceinline__ void adj_main_general_block(const double *__restrict_
   const int EB = a.EB;
   double *lops = lds;
   double *lU = lops + S::NOPS_PAD;
-  double *lR = lU + EB * V * nS;
+  double *lR = lU + EB * L::U;
   double *lGB = lR + EB * L::R;
   const long e0 = bid * EB;
   const long neb = min((long)EB, (long)a.E - e0);
   const int tid = threadIdx.x, el = tid / nS, t = tid - el * nS;
   const long e = e0 + el;
   const bool valid = el < neb;
-  const double *u = lU + el * V * nS;
+  const double *u = lU + el * L::U;
   double *c = lR + el * L::R, *T = c, *to = c;
-  double *gb = lGB + el * D * V * nS;
+  double *gb = lGB + el * L::GB;
   StageRegs<D, N> sr;
   stage_U_load<D, N>(U, a, e0, neb, sr);
   if (valid) {
 #pragma unroll
     for (int v = 0; v < V; v++) gb[v * nS + t] = w[(e * V + v) * nS + t];
   }
-  stage_U_store<D, N>(U, a, lops, lU, e0, neb, V * nS, sr);
+  stage_U_store<D, N>(U, a, lops, lU, e0, neb, L::U, sr);
   __syncthreads();
   const int ia = t % N, ib = (t / N) % N, ic = (D == 3) ? t / (N * N) : 0;
   const double beta = a.ldg_b;

@@ -63,6 +63,14 @@ struct Shape {
   // workgroup size bound of the per-shape kernels: 256 threads, or one element's points
   // rounded up to whole waves where an element has more (hexes of order 6 to 8)
   static constexpr int kThreads = (nS > kMaxThreads) ? ((nS + 63) / 64) * 64 : kMaxThreads;
+  // LDS stride of per-element blocks of x doubles.  A wave's 64-bit LDS access goes 16 lanes at
+  // a time over 32 banks, so doubles a multiple of 16 apart collide; with strides that are nS
+  // modulo 16, lanes of neighbouring elements continue one run of banks (where a workgroup can
+  // hold two elements at all).  Blocks back to back put up to 16 lanes on one bank for quads
+  // p=1: Navier-Stokes residual of 300x301 of them 42.2 us, padded 35.6; 256^2 quads p=4 114
+  // / 111, V-cycle of 128^2 quads p=4 458 / 454.  (Planes of hexes p=3 padded to 19, so that
+  // the face phase's line gathers hit distinct banks too, gained nothing: 64^3 1525 / 1530.)
+  static constexpr int ele(int x) { return 2 * nS > kMaxThreads ? x : x + ((nS - x) % 16 + 16) % 16; }
 };
 
 // The hardware dispatches workgroup b of a grid to XCD b % 8 (each XCD has its own L2).
@@ -721,10 +729,10 @@ __device__ __forceinline__ void extrapolate_block(const double *__restrict__ U, 
     const int f = t + k * nS;
     slot[k] = (a.trace_sel && el < neb && f < nF) ? nbr_slot<D, N>(a.nbr[e * nF + f]) : -1;
   }
-  stage_U<D, N>(U, a, lops, lU, e0, neb, V * nS);
+  stage_U<D, N>(U, a, lops, lU, e0, neb, S::ele(V * nS));
   __syncthreads();
   if (el >= neb) return;
-  const double *u = lU + el * V * nS;
+  const double *u = lU + el * S::ele(V * nS);
   const int owner = (a.ldg_b == 0.5) ? 0 : 1;
 #pragma unroll
   for (int k = 0; k < S::FPT; k++) {
@@ -846,7 +854,7 @@ __device__ __forceinline__ void gradient_block(const double *__restrict__ U, dou
                                                const KArgs &a, long bid) {
   using S = Shape<D, N>;
   constexpr int nS = S::nS, nF = S::nF, V = S::V;
-  constexpr int W = (V * nS + V * nF > D * V * nS) ? V * nS + V * nF : D * V * nS;
+  constexpr int W = S::ele((V * nS + V * nF > D * V * nS) ? V * nS + V * nF : D * V * nS);
   extern __shared__ double lds[];
   double *lops = lds;
   double *lW = lds + S::NOPS_PAD;
@@ -925,8 +933,9 @@ __device__ __forceinline__ void divergence_block(const double *U, double *__rest
   const int EB = a.EB;
   double *lops = lds;
   double *lU = lops + S::NOPS_PAD;
-  double *lC = lU + EB * V * nS;
-  double *lG = lC + EB * V * nF;  // gradient (viscous), then the transformed flux
+  constexpr int WU = S::ele(V * nS), WC = S::ele(V * nF), WG = S::ele(D * V * nS);
+  double *lC = lU + EB * WU;
+  double *lG = lC + EB * WC;  // gradient (viscous), then the transformed flux
   const long e0 = bid * EB;
   const long neb = min((long)EB, (long)a.E - e0);
   const int tid = threadIdx.x, el = tid / nS, t = tid - el * nS;
@@ -975,14 +984,14 @@ __device__ __forceinline__ void divergence_block(const double *U, double *__rest
         for (int v = 0; v < V; v++) pUs[k][v] = a.Utr[(ep * V + v) * nF + fp];
       }
     }
-    stage_U_store<D, N>(U, a, lops, lU, e0, neb, V * nS, sr);
+    stage_U_store<D, N>(U, a, lops, lU, e0, neb, WU, sr);
   } else {
-    stage_U<D, N>(U, a, lops, lU, e0, neb, V * nS);
+    stage_U<D, N>(U, a, lops, lU, e0, neb, WU);
   }
   __syncthreads();
-  const double *u = lU + el * V * nS;
-  double *c = lC + el * V * nF;
-  double *g_l = lG + el * D * V * nS;
+  const double *u = lU + el * WU;
+  double *c = lC + el * WC;
+  double *g_l = lG + el * WG;
   if (VISC) {
     if (valid) common_solution<D, N>(a, lops, u, c, e, t);
     __syncthreads();
@@ -1167,9 +1176,9 @@ __device__ __forceinline__ void divergence_block(const double *U, double *__rest
   }
   // the new state's full trace for the next stage, into a buffer other than the Utr this
   // launch reads; the element's U block is no longer read
-  if (a.rk.mode == 1 && a.rk.trace) rk_trace<D, N>(a, lops, lU + el * V * nS, e, t, valid, unew, -1);
+  if (a.rk.mode == 1 && a.rk.trace) rk_trace<D, N>(a, lops, lU + el * WU, e, t, valid, unew, -1);
   // p-multigrid transfers (the U block is still the staged state; lG is free)
-  if (a.rk.pmgRc || a.rk.pmgUf) pmg_epilogue<D, N>(a, lops, lU + el * V * nS, g_l, e, t, valid, res, unew);
+  if (a.rk.pmgRc || a.rk.pmgUf) pmg_epilogue<D, N>(a, lops, lU + el * WU, g_l, e, t, valid, res, unew);
 }
 
 // Occupancy target of the divergence kernel: the general-beta hex p=3 Rusanov kernel fits
@@ -1242,12 +1251,12 @@ __device__ __forceinline__ void visc_onesided_block(const double *__restrict__ U
   constexpr int owner = (BM == 2) ? 1 : 0;  // slot that forms the convective flux (and, beta = +-1/2, whose gradient enters)
   // one LDS region per element holds the common solution, then (after a barrier) the
   // gradient, then the transformed flux
-  constexpr int W = (V * nF > D * V * nS) ? V * nF : D * V * nS;
+  constexpr int WU = S::ele(V * nS), W = S::ele((V * nF > D * V * nS) ? V * nF : D * V * nS);
   extern __shared__ double lds[];
   const int EB = a.EB;
   double *lops = lds;
   double *lU = lops + S::NOPS_PAD;
-  double *lW = lU + EB * V * nS;
+  double *lW = lU + EB * WU;
   const long e0 = bid * EB;
   const long neb = min((long)EB, (long)a.E - e0);
   const int tid = threadIdx.x, el = tid / nS, t = tid - el * nS;
@@ -1293,7 +1302,7 @@ __device__ __forceinline__ void visc_onesided_block(const double *__restrict__ U
     }
     // the staged block has arrived with the entries (loads return in order): its registers
     // are free for the lines
-    stage_U_store<D, N>(U, a, lops, lU, e0, neb, V * nS, sr);
+    stage_U_store<D, N>(U, a, lops, lU, e0, neb, WU, sr);
     PartnerLine<D, N> pl[self ? S::FPT : 1];
     double x[S::FPT][V];
 #pragma unroll
@@ -1346,9 +1355,9 @@ __device__ __forceinline__ void visc_onesided_block(const double *__restrict__ U
       a.Utr[(e * V + v) * nF + f] = x[v];
     }
   }
-  if constexpr (BM != 0) stage_U_store<D, N>(U, a, lops, lU, e0, neb, V * nS, sr);
+  if constexpr (BM != 0) stage_U_store<D, N>(U, a, lops, lU, e0, neb, WU, sr);
   __syncthreads();
-  const double *u = lU + el * V * nS;
+  const double *u = lU + el * WU;
   double *g_l = lW + el * W;
   // common solution: beta = +-1/2 the non-owner side's state, so this element's own trace
   // where the partner owns the face; else both sides' traces mixed
@@ -1541,7 +1550,7 @@ __device__ __forceinline__ void face_correction_block(double *__restrict__ divF,
   constexpr int owner = (BM == 2) ? 1 : 0;
   // per-element LDS block: the common fluxes (V * nF), then the new state (V * nS) when the
   // RK update writes the next trace
-  constexpr int W = V * (nF > nS ? nF : nS);
+  constexpr int W = S::ele(V * (nF > nS ? nF : nS));
   extern __shared__ double lds[];
   const int EB = a.EB;
   double *lops = lds;
@@ -1716,26 +1725,26 @@ struct AdjPtrs {
 template <int D, int N>
 size_t lds_per_element(Op op, bool viscous) {
   using S = Shape<D, N>;
-  constexpr size_t kUC = (size_t)S::V * S::nS + S::V * S::nF, kG = (size_t)D * S::V * S::nS;
+  constexpr int VS = S::V * S::nS, VF = S::V * S::nF, G = D * VS;
   size_t per_ele = 0;
   switch (op) {
     case Op::Extrap:
-    case Op::ExtrapPartner: per_ele = (size_t)S::V * S::nS; break;
-    case Op::Grad: per_ele = kUC > kG ? kUC : kG; break;
-    case Op::Div: per_ele = kUC + kG; break;
+    case Op::ExtrapPartner: per_ele = S::ele(VS); break;
+    case Op::Grad: per_ele = S::ele(VS + VF > G ? VS + VF : G); break;
+    case Op::Div: per_ele = S::ele(VS) + S::ele(VF) + S::ele(G); break;
     case Op::OneSided:
     case Op::OneSidedFromTrace:
     case Op::BothSides:
     case Op::BothSidesFromTrace:
-      per_ele = (size_t)S::V * S::nS + (S::V * S::nF > (int)kG ? S::V * S::nF : kG);
+      per_ele = S::ele(VS) + S::ele(VF > G ? VF : G);
       break;
     case Op::FaceCorr:
-    case Op::FaceCorrBoth: per_ele = (size_t)S::V * (S::nF > S::nS ? S::nF : S::nS); break;
-    case Op::AdjPrep: per_ele = (size_t)S::V * S::nS; break;
+    case Op::FaceCorrBoth: per_ele = S::ele(VF > VS ? VF : VS); break;
+    case Op::AdjPrep: per_ele = VS; break;
     case Op::AdjMain:
       per_ele = viscous ? (size_t)AdjLds<D, N, true>::per_ele : (size_t)AdjLds<D, N, false>::per_ele;
       break;
-    case Op::AdjGather: per_ele = (size_t)S::V * S::nF; break;
+    case Op::AdjGather: per_ele = S::ele(VF); break;
     case Op::AdjFace: per_ele = 0; break;
     case Op::AdjMainGen: per_ele = (size_t)AdjGenLds<D, N>::per_ele; break;
   }
