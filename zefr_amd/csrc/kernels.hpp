@@ -1262,20 +1262,34 @@ __device__ __forceinline__ void visc_onesided_block(const double *__restrict__ U
   const int tid = threadIdx.x, el = tid / nS, t = tid - el * nS;
   const long e = e0 + el;
   const bool valid = el < neb;
-  // Work item k of an element is its k-th owned flux point: thread t takes k = t in the
-  // prologue and again in the face phase, so the partner's trace there stays in its
-  // registers (half of the flux points are owned on average, so the items beyond the first
-  // nS are rare for N >= 3; their traces are parked in Utr at this element's own points,
-  // which nothing else reads).  The staging loads are issued first and the partner's values
-  // before any is consumed; with SELF they are its solution line through the point (no
-  // trace launch runs before this kernel), otherwise its trace from Utr.
+  // Work item k of an element is its k-th owned flux point.  Quads of N >= 5 points per
+  // direction own about 2 N of their 4 N <= N^2 flux points, and the items of an element on its
+  // own points' lanes kept every wave busy in the longest phase with 2 / N of its lanes.  There
+  // the first H = 2 N items of all the workgroup's elements are dealt to its threads in a row,
+  // then the others (of elements that own more faces): a thread has one item at most, (fe, fk)
+  // its element and item, and waves without any skip the phase.  Elsewhere items stay on their
+  // element's lanes, nS apart: hexes have 3 / N of the lanes busy and lose as much by the second
+  // element index (64^3 p=3 Roe 1530 / 1580 us, 13x11x17 p=5 71 / 77), quads p=3 gain nothing
+  // (256^2 67 / 70).  In lanes / in a row: 256^2 quads p=4 112 / 105 us, with Roe 115 / 112;
+  // 96x100 23.0 / 21.8; 200x201 p=5 106 / 97; 150x151 p=6 90 / 80; 24^2 p=6 11.7 / 11.7.
+  // A thread takes its item in the prologue and again in the face phase, so the partner's trace
+  // there stays in its registers (a second item, nS further, is rare for N >= 3; its trace is
+  // parked in Utr at the element's own point, which nothing else reads).  The staging loads are issued first and
+  // the partner's values before any is consumed; with SELF they are its solution line through
+  // the point (no trace launch runs before this kernel), otherwise its trace from Utr.
   constexpr bool self = SELF;
+  constexpr bool kRow = BM != 0 && D == 2 && N >= 5 && nS % 64 != 0;
+  constexpr int H = D * S::nFF, Q = kRow ? nF : nS;
   StageRegs<D, N> sr;
   stage_U_load<D, N>(U, a, e0, neb, sr);
-  const unsigned mask = valid ? owned_faces<D, N>(a.nbr + e * nF, owner) : 0u;
+  const int half = (kRow && tid >= EB * H) ? 1 : 0, ti = tid - half * EB * H;
+  const int fe = kRow ? ti / H : el, fk = kRow ? ti - fe * H + half * H : t;
+  const bool fvalid = kRow ? fe < neb : valid;
+  const long ef = kRow ? e0 + fe : e;
+  const unsigned mask = fvalid ? owned_faces<D, N>(a.nbr + ef * nF, owner) : 0u;
   const unsigned owned = face_list<D>(mask), unowned = face_list<D>(~mask);
   const int cnt = __popc(mask) * S::nFF;
-  double *c = lW + el * W;
+  double *c = lW + el * W, *cf = lW + fe * W;
   double cp[V];
   // general beta: the items are all flux points, the owned ones first, and the partner's
   // trace is needed at each (nothing is parked: with SELF = false partners read every entry
@@ -1285,7 +1299,7 @@ __device__ __forceinline__ void visc_onesided_block(const double *__restrict__ U
   };
   auto partner = [&](int f, double *x) {
     long ep; int sl, fp;
-    unpack_nbr<D, N>(a.nbr[e * nF + f], ep, sl, fp);
+    unpack_nbr<D, N>(a.nbr[ef * nF + f], ep, sl, fp);
     if constexpr (self) {
       partner_trace<D, N>(U, a.ops, ep, fp, x);
     } else {
@@ -1297,8 +1311,8 @@ __device__ __forceinline__ void visc_onesided_block(const double *__restrict__ U
     unsigned nb[S::FPT];
 #pragma unroll
     for (int k = 0; k < S::FPT; k++) {
-      const int i = t + k * nS;
-      nb[k] = (valid && i < nF) ? a.nbr[e * nF + item_fpt(i)] : 0u;
+      const int i = fk + k * nS;
+      nb[k] = (fvalid && i < nF) ? a.nbr[ef * nF + item_fpt(i)] : 0u;
     }
     // the staged block has arrived with the entries (loads return in order): its registers
     // are free for the lines
@@ -1307,7 +1321,7 @@ __device__ __forceinline__ void visc_onesided_block(const double *__restrict__ U
     double x[S::FPT][V];
 #pragma unroll
     for (int k = 0; k < S::FPT; k++) {
-      if (!valid || t + k * nS >= nF) continue;
+      if (!fvalid || fk + k * nS >= nF) continue;
       long ep; int sl, fp;
       unpack_nbr<D, N>(nb[k], ep, sl, fp);
       if constexpr (self) {
@@ -1319,20 +1333,20 @@ __device__ __forceinline__ void visc_onesided_block(const double *__restrict__ U
     }
 #pragma unroll
     for (int k = 0; k < S::FPT; k++) {
-      const int i = t + k * nS;
-      if (!valid || i >= nF) continue;
+      const int i = fk + k * nS;
+      if (!fvalid || i >= nF) continue;
       if constexpr (self) partner_line_reduce<D, N>(pl[k], x[k]);
       const int f = item_fpt(i);
 #pragma unroll
-      for (int v = 0; v < V; v++) c[v * nF + f] = x[k][v];
+      for (int v = 0; v < V; v++) cf[v * nF + f] = x[k][v];
     }
 #pragma unroll
     for (int v = 0; v < V; v++) cp[v] = x[0][v];
   }
-  if (BM != 0 && t < cnt && valid) {
-    const int f = list_fpt<D, N>(owned, t);
+  if (BM != 0 && fk < cnt && fvalid) {
+    const int f = list_fpt<D, N>(owned, fk);
     long ep; int sl, fp;
-    unpack_nbr<D, N>(a.nbr[e * nF + f], ep, sl, fp);
+    unpack_nbr<D, N>(a.nbr[ef * nF + f], ep, sl, fp);
     if constexpr (self) {
       PartnerLine<D, N> pl;
       partner_line_load<D, N>(U, a.ops, ep, fp, pl);
@@ -1342,49 +1356,49 @@ __device__ __forceinline__ void visc_onesided_block(const double *__restrict__ U
       for (int v = 0; v < V; v++) cp[v] = a.Utr[(ep * V + v) * nF + fp];
     }
 #pragma unroll
-    for (int v = 0; v < V; v++) c[v * nF + f] = cp[v];
+    for (int v = 0; v < V; v++) cf[v * nF + f] = cp[v];
   }
 #pragma unroll 1
-  for (int k = t + nS; BM != 0 && k < cnt; k += nS) {
+  for (int k = fk + Q; BM != 0 && k < cnt; k += Q) {
     const int f = list_fpt<D, N>(owned, k);
     double x[V];
     partner(f, x);
 #pragma unroll
     for (int v = 0; v < V; v++) {
-      c[v * nF + f] = x[v];
-      a.Utr[(e * V + v) * nF + f] = x[v];
+      cf[v * nF + f] = x[v];
+      a.Utr[(ef * V + v) * nF + f] = x[v];
     }
   }
   if constexpr (BM != 0) stage_U_store<D, N>(U, a, lops, lU, e0, neb, WU, sr);
   __syncthreads();
-  const double *u = lU + el * WU;
-  double *g_l = lW + el * W;
+  const double *u = lU + el * WU, *uf = lU + fe * WU;
+  double *g_l = c, *gf = cf;
   // common solution: beta = +-1/2 the non-owner side's state, so this element's own trace
   // where the partner owns the face; else both sides' traces mixed
-  if (BM == 0 && valid) {
-    for (int k = t; k < nF; k += nS) {
+  if (BM == 0 && fvalid) {
+    for (int k = fk; k < nF; k += Q) {
       const int f = item_fpt(k);
       int dim, side, base, str;
       fpt_info<D, N>(f, dim, side, base, str);
       const double *lE = tab_lE<N>(lops, side);
 #pragma unroll
       for (int v = 0; v < V; v++) {
-        const double own = line_extrap<N>(lE, u + v * nS, base, str), par = c[v * nF + f];
+        const double own = line_extrap<N>(lE, uf + v * nS, base, str), par = cf[v * nF + f];
         const double l = (k < cnt) ? own : par, r = (k < cnt) ? par : own;
-        c[v * nF + f] = 0.5 * (l + r) - a.ldg_b * (l - r);
+        cf[v * nF + f] = 0.5 * (l + r) - a.ldg_b * (l - r);
       }
     }
   }
-  if (BM != 0 && valid) {
+  if (BM != 0 && fvalid) {
     const int rest = nF - cnt;
 #pragma unroll 1
-    for (int k = t; k < rest; k += nS) {
+    for (int k = fk; k < rest; k += Q) {
       const int f = list_fpt<D, N>(unowned, k);
       int dim, side, base, str;
       fpt_info<D, N>(f, dim, side, base, str);
       const double *lE = tab_lE<N>(lops, side);
 #pragma unroll
-      for (int v = 0; v < V; v++) c[v * nF + f] = line_extrap<N>(lE, u + v * nS, base, str);
+      for (int v = 0; v < V; v++) cf[v * nF + f] = line_extrap<N>(lE, uf + v * nS, base, str);
     }
   }
   __syncthreads();
@@ -1407,20 +1421,20 @@ __device__ __forceinline__ void visc_onesided_block(const double *__restrict__ U
   // common normal flux (unscaled) at the owned flux points -> Ftr; general beta: this side's
   // share of it at every flux point (the convective flux and the penalty at owned ones, this
   // side's viscous flux with its weight at all)
-  if (valid) {
+  if (fvalid) {
 #pragma unroll 1
-    for (int k = t; k < (BM == 0 ? nF : cnt); k += nS) {
+    for (int k = fk; k < (BM == 0 ? nF : cnt); k += Q) {
       const int f = item_fpt(k);  // face-major: neighbouring lanes, neighbouring points
       int dim, side, base, str;
       fpt_info<D, N>(f, dim, side, base, str);
       const double *lE = tab_lE<N>(lops, side);
-      const double *fg = a.fgeo + e * (D + 1) * nF + f;
+      const double *fg = a.fgeo + ef * (D + 1) * nF + f;
       double n[D];
 #pragma unroll
       for (int d = 0; d < D; d++) n[d] = fg[d * nF];
       double Uo[V], Up[V];
 #pragma unroll
-      for (int v = 0; v < V; v++) Uo[v] = line_extrap<N>(lE, u + v * nS, base, str);
+      for (int v = 0; v < V; v++) Uo[v] = line_extrap<N>(lE, uf + v * nS, base, str);
       // the convective flux and the LDG penalty first, so that their temporaries and the
       // partner's state are dead before the gradient's lines are gathered (Roe in the other
       // order needs ~350 registers)
@@ -1428,14 +1442,14 @@ __device__ __forceinline__ void visc_onesided_block(const double *__restrict__ U
 #pragma unroll
       for (int v = 0; v < V; v++) Fo[v] = 0.0;
       if (BM != 0 || k < cnt) {
-        if (k == t) {
+        if (k == fk) {
 #pragma unroll
           for (int v = 0; v < V; v++) Up[v] = cp[v];
         } else if (BM == 0) {
           partner(f, Up);
         } else {
 #pragma unroll
-          for (int v = 0; v < V; v++) Up[v] = a.Utr[(e * V + v) * nF + f];
+          for (int v = 0; v < V; v++) Up[v] = a.Utr[(ef * V + v) * nF + f];
         }
         if (owner == 0) {
           conv_common_flux<D, FC>(Uo, Up, n, a, Fo);
@@ -1453,7 +1467,7 @@ __device__ __forceinline__ void visc_onesided_block(const double *__restrict__ U
       visc_normal<D>(Uo, [&](int j, double *dUj) {
 #pragma unroll
         for (int v = 0; v < V; v++) {
-          dUj[v] = line_extrap<N>(lE, g_l + (j * V + v) * nS, base, str);
+          dUj[v] = line_extrap<N>(lE, gf + (j * V + v) * nS, base, str);
           asm volatile("" : "+v"(dUj[v]) : : "memory");  // formed here, before the next line is loaded
         }
       }, n, a, G);
@@ -1462,7 +1476,7 @@ __device__ __forceinline__ void visc_onesided_block(const double *__restrict__ U
 #pragma unroll
       for (int v = 0; v < V; v++) Fo[v] += wt * G[v];
 #pragma unroll
-      for (int v = 0; v < V; v++) __builtin_nontemporal_store(Fo[v], &a.Ftr[(e * V + v) * nF + f]);
+      for (int v = 0; v < V; v++) __builtin_nontemporal_store(Fo[v], &a.Ftr[(ef * V + v) * nF + f]);
     }
   }
   __syncthreads();  // the gradient field is consumed
