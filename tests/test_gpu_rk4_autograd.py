@@ -90,3 +90,32 @@ def test_general_path_kept():
         assert not isinstance(Y.grad_fn, RK4Step._backward_cls)
         assert torch.isfinite(torch.autograd.grad(Y.sum(), U)[0]).all()
     assert torch.isfinite(torch.autograd.grad(rk4_step(z, U, 1e-3, dj).sum(), dj)[0]).all()
+
+
+def test_saved_tensor_hooks_and_dual_detJ():
+    """Saved tensors that hooks hand back in another layout give the same gradient, one that comes
+    back on the host is refused, and a detJ with a tangent takes the tensor expressions."""
+    import torch
+    from torch.autograd import forward_ad, graph
+    from zefr_amd.autograd import RK4Step, _fusable, device_field, rk4_step
+    z = solver((4, 3), 2, True)
+    detJ, U0 = device_field(z, "jaco_det_spts"), field(z, 1)
+    grads = []
+    for hooks in (None, (lambda x: x, lambda x: x.transpose(0, -1).contiguous().transpose(0, -1))):
+        U = U0.clone().requires_grad_()
+        if hooks:
+            with graph.saved_tensors_hooks(*hooks):
+                Y = rk4_step(z, U, 1e-3, detJ)
+        else:
+            Y = rk4_step(z, U, 1e-3, detJ)
+        assert isinstance(Y.grad_fn, RK4Step._backward_cls)
+        grads.append(torch.autograd.grad(Y.square().sum(), U)[0])
+    assert torch.equal(*grads)
+    U = U0.clone().requires_grad_()
+    with graph.saved_tensors_hooks(lambda x: x, lambda x: x.cpu() if x.shape == detJ.shape else x):
+        Y = rk4_step(z, U, 1e-3, detJ)
+    with pytest.raises(RuntimeError, match="detJ"):
+        torch.autograd.grad(Y.sum(), U)
+    with forward_ad.dual_level():
+        assert _fusable(z, U0, 1e-3, detJ, None)
+        assert not _fusable(z, U0, 1e-3, forward_ad.make_dual(detJ, torch.ones_like(detJ)), None)

@@ -134,9 +134,12 @@ class RK4Step(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, g):
-        U, X2, X3, X4, detJ = ctx.saved_tensors
+        U, X2, X3, X4, detJ = ctx.saved_tensors  # saved-tensor hooks may return other layouts
+        if not (detJ.is_cuda and detJ.dtype == torch.float64 and detJ.numel() == g.shape[0] * g.shape[2]):
+            raise RuntimeError("rk4_step: the saved detJ came back on another device, or of another type or size")
         with torch.no_grad():
-            v = RK4Step._reverse(ctx.z, ctx.dt, detJ, (U.contiguous(), X2, X3, X4), g.contiguous())
+            v = RK4Step._reverse(ctx.z, ctx.dt, detJ.contiguous(), [x.contiguous() for x in (U, X2, X3, X4)],
+                                 g.contiguous())
         if torch.is_grad_enabled():  # create_graph: v depends on g through the identity; the VJPs are constants
             v = g + (v - g.detach())
         return v, None, None, None
@@ -171,7 +174,8 @@ def _fusable(z, U, dt, detJ, mu):
     return (mu is None and type(dt) in (int, float) and type(U) in (torch.Tensor, torch.nn.Parameter)
             and type(detJ) is torch.Tensor and U.dim() == 3 and detJ.shape == (U.shape[0], 1, U.shape[2])
             and detJ.dtype == torch.float64 and U.dtype == torch.float64 and detJ.is_cuda and U.is_cuda
-            and detJ.device == U.device and detJ.is_contiguous() and not detJ.requires_grad)
+            and detJ.device == U.device and detJ.is_contiguous() and not detJ.requires_grad
+            and torch.autograd.forward_ad.unpack_dual(detJ).tangent is None)
 
 
 def rk4_step(z, U, dt, detJ=None, mu=None):
