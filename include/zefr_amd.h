@@ -195,7 +195,8 @@ int zefr_time_residual_kernels(zefr_t *z, int reps, double *ms_out);
  * get_u_spts_d) on the caller's `stream` (NULL: the null stream), with the kernels of
  * compute_residual (src/solver.cpp:1494-1645) but without touching the solver's state.
  * It uses the solver's trace scratch: do not overlap it with other work of the solver
- * (its own stream is non-blocking, so synchronise in between). */
+ * (its own stream is non-blocking, so synchronise in between).  With an LDG beta other than
+ * +-1/2 divF may be U; otherwise the two must not overlap. */
 int zefr_residual_at(zefr_t *z, const double *U, double *divF, void *stream);
 /* v = (dR/dU)^T w at U (all device pointers, layout [E][V][nS]) on `stream` (NULL: the
  * null stream): the residual's vector-Jacobian product (new; no reference counterpart).

@@ -421,6 +421,16 @@ void FRSolver::compute_residual(unsigned stage, int color) {
 
 void FRSolver::residual_at(const double *U, double *divF, hipStream_t st) {
   need_device(*this);
+  if (input->viscous && !onesided() && U == divF) {
+    // in place: the first of the two launches below reads the partners' states while it writes
+    // the volume part of divF; of these three only the last one writes, and it reads its own
+    // elements' state and the traces
+    const auto d0 = eles->desc(*input, 0), d1 = eles->desc(*input, 1), d2 = eles->desc(*input, 2);
+    status_or_throw(zfr_extrapolate(&d0, U, st));
+    status_or_throw(zfr_gradient(&d1, U, nullptr, st));
+    status_or_throw(zfr_divergence(&d2, U, divF, st));
+    return;
+  }
   if (input->viscous) viscous_flux(eles->desc(*input, 1), U, divF, st);
   last_launch(eles->desc(*input, 2), U, divF, nullptr, st);
 }
