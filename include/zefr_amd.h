@@ -315,7 +315,7 @@ int zfr_divergence(const zfr_ele_desc_t *d, const double *U, double *divF, void 
 int zfr_gradient_flux(const zfr_ele_desc_t *d, const double *U, double *divF, void *stream);
 /* The same, reading the partner traces from d->Utr at the partner's points instead (as
  * written by zfr_extrapolate_partner, or by the previous RK stage's fused update with
- * trace_out = d->Utr); used for RK stages 1.. whose trace is already on the device. */
+ * trace_out = d->Utr).  d->Utr is only read. */
 int zfr_gradient_flux_traced(const zfr_ele_desc_t *d, const double *U, double *divF, void *stream);
 /* Elements::compute_divF_fpts (src/elements.cpp:1476-1501) on that path:
  * divF += oppDiv_fpts Fcomm with Fcomm = owner's Ftr * signed dA of this side. */

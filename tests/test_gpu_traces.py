@@ -1,0 +1,44 @@
+"""The solution traces that launches read from Utr or write for the next one."""
+
+from __future__ import annotations
+
+import ctypes as C
+
+import pytest
+
+from ele_block import Block, ok, ptr
+from zefr_amd import _lib
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("D,order,first", [(2, 0, 3), (2, 1, 3), (3, 0, 5), (3, 1, 4), (3, 2, 6), (2, 4, 3), (3, 3, 3),
+                                           (3, 6, 3)])
+@pytest.mark.parametrize("beta,flux", [(0.5, 0), (-0.5, 2)])
+def test_traced_gradient_flux_only_reads_the_trace(D, order, first, beta, flux):
+    """The whole trace is as zfr_extrapolate left it, also at the points of elements that own
+    more flux points than they have solution points, and the results are zfr_gradient_flux's."""
+    import torch
+    L, b = _lib.lib(), Block(D, order, first=first)
+    for tile in (0, 3):
+        d, out = b.desc(beta=beta, flux=flux, tile=tile), []
+        for traced in (False, True):
+            dF = b.field()
+            b.Ftr.zero_()
+            if traced:
+                b.Utr.fill_(7.0)
+                torch.cuda.synchronize()
+                ok(L.zfr_extrapolate(C.byref(d), ptr(b.U), None))
+                torch.cuda.synchronize()
+                before = b.Utr.clone()
+                torch.cuda.synchronize()
+                ok(L.zfr_gradient_flux_traced(C.byref(d), ptr(b.U), ptr(dF), None))
+                torch.cuda.synchronize()
+                assert torch.equal(b.Utr, before)
+            else:
+                torch.cuda.synchronize()
+                ok(L.zfr_gradient_flux(C.byref(d), ptr(b.U), ptr(dF), None))
+                torch.cuda.synchronize()
+            out.append((dF, b.Ftr.clone()))
+        assert torch.isfinite(out[0][0]).all() and out[0][1].abs().sum() > 0
+        assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])

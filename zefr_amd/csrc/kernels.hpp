@@ -1239,10 +1239,10 @@ struct OneSidedWaves {
 };
 
 // SELF: extrapolate the partner traces this element needs from the partner's U (no trace
-// launch before this kernel; they are parked in Utr at this element's own owned points
-// for the face phase); otherwise read them from Utr at the partner's points (written by a
-// trace launch or by the previous RK stage's update).  A template parameter: as a
-// run-time branch the two prologues together spill the hex p=3 kernel.
+// launch before this kernel); otherwise read them from Utr at the partner's points (written
+// by a trace launch or by the previous RK stage's update), which this kernel then leaves as
+// it is.  A template parameter: as a run-time branch the two prologues together spill the
+// hex p=3 kernel.
 template <int D, int N, int BM, int FC, bool SELF>
 __device__ __forceinline__ void visc_onesided_block(const double *__restrict__ U, double *__restrict__ divF,
                                                     const KArgs &a, long bid) {
@@ -1272,11 +1272,13 @@ __device__ __forceinline__ void visc_onesided_block(const double *__restrict__ U
   // element index (64^3 p=3 Roe 1530 / 1580 us, 13x11x17 p=5 71 / 77), quads p=3 gain nothing
   // (256^2 67 / 70).  In lanes / in a row: 256^2 quads p=4 112 / 105 us, with Roe 115 / 112;
   // 96x100 23.0 / 21.8; 200x201 p=5 106 / 97; 150x151 p=6 90 / 80; 24^2 p=6 11.7 / 11.7.
-  // A thread takes its item in the prologue and again in the face phase, so the partner's trace
-  // there stays in its registers (a second item, nS further, is rare for N >= 3; its trace is
-  // parked in Utr at the element's own point, which nothing else reads).  The staging loads are issued first and
-  // the partner's values before any is consumed; with SELF they are its solution line through
-  // the point (no trace launch runs before this kernel), otherwise its trace from Utr.
+  // A thread takes its item in the prologue and again in the face phase, so with SELF the
+  // partner's trace there stays in its registers (a second item, nS further, is rare for
+  // N >= 3; its trace is parked in Utr at the element's own point, which nothing else reads).
+  // The staging loads are issued first and the partner's values before any is consumed; with
+  // SELF they are its solution line through the point (no trace launch runs before this
+  // kernel), otherwise its trace from Utr, which is only read: the face phase reads it there
+  // again (held instead, hexes p=6 take 146 VGPRs for 126).
   constexpr bool self = SELF;
   constexpr bool kRow = BM != 0 && D == 2 && N >= 5 && nS % 64 != 0;
   constexpr int H = D * S::nFF, Q = kRow ? nF : nS;
@@ -1292,8 +1294,8 @@ __device__ __forceinline__ void visc_onesided_block(const double *__restrict__ U
   double *c = lW + el * W, *cf = lW + fe * W;
   double cp[V];
   // general beta: the items are all flux points, the owned ones first, and the partner's
-  // trace is needed at each (nothing is parked: with SELF = false partners read every entry
-  // of Utr; the few owned items beyond the first nS fetch it again in the face phase)
+  // trace is needed at each (nothing is parked: the few owned items beyond the first nS fetch
+  // it again in the face phase)
   auto item_fpt = [&](int k) {
     return (BM == 0 && k >= cnt) ? list_fpt<D, N>(unowned, k - cnt) : list_fpt<D, N>(owned, k);
   };
@@ -1366,7 +1368,7 @@ __device__ __forceinline__ void visc_onesided_block(const double *__restrict__ U
 #pragma unroll
     for (int v = 0; v < V; v++) {
       cf[v * nF + f] = x[v];
-      a.Utr[(ef * V + v) * nF + f] = x[v];
+      if (self) a.Utr[(ef * V + v) * nF + f] = x[v];
     }
   }
   if constexpr (BM != 0) stage_U_store<D, N>(U, a, lops, lU, e0, neb, WU, sr);
@@ -1442,10 +1444,10 @@ __device__ __forceinline__ void visc_onesided_block(const double *__restrict__ U
 #pragma unroll
       for (int v = 0; v < V; v++) Fo[v] = 0.0;
       if (BM != 0 || k < cnt) {
-        if (k == fk) {
+        if (self && k == fk) {
 #pragma unroll
           for (int v = 0; v < V; v++) Up[v] = cp[v];
-        } else if (BM == 0) {
+        } else if (BM == 0 || !self) {
           partner(f, Up);
         } else {
 #pragma unroll
