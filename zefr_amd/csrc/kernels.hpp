@@ -948,32 +948,21 @@ __device__ __forceinline__ void divergence_block(const double *U, double *__rest
   // them, they were 2 FPT + 1, and on small meshes a launch is little else.  Out-of-range
   // threads and points load a neighbour's data (in bounds) instead of branching.  (29x31x27
   // hexes p=2, RK44 step 246 -> 232 us; 128^2 quads p=4, V-cycle 520 -> 495.)
+  // Not so in hexes of order 6 to 8 (one element and 6 to 12 waves per workgroup, one flux
+  // point at most per thread): there the lines held beside all the rest cost a wave of three
+  // (p=6, 172 registers) or 42 spills (p=8), and whole waves have no flux point to load for.
+  // They take the partner's line first and branch.  Residual, all ahead / line first: 8x7x7
+  // hexes p=8 42.2 / 29.6 us, 15x13x14 252 / 172; 10x9x10 p=6 33.3 / 32.0, 19x17x18 188 / 159.
   constexpr int PF = VISC ? 1 : S::FPT;
   double pUs[PF][V], pn[PF][D], pdA[PF], pij[D][D], pdet = 1.0;
   int psl[PF];
   RkPre<D> pre;
+  constexpr bool ahead = nS <= kMaxThreads;
   if constexpr (!VISC) {
     const long ec = valid ? e : e0;
     StageRegs<D, N> sr;
-    stage_U_load<D, N>(U, a, e0, neb, sr);
     unsigned nb[PF];
-#pragma unroll
-    for (int k = 0; k < PF; k++) {
-      const int f = t + k * nS;
-      nb[k] = a.nbr[ec * nF + (f < nF ? f : 0)];
-    }
-#pragma unroll
-    for (int k = 0; k < PF; k++) {
-      const int f = t + k * nS;
-      const double *fg = a.fgeo + ec * (D + 1) * nF + (f < nF ? f : 0);
-#pragma unroll
-      for (int d = 0; d < D; d++) pn[k][d] = fg[d * nF];
-      pdA[k] = fg[D * nF];
-    }
-    load_metric<D>(a, ec, t, nS, pij, pdet, false);
-    rk_prefetch<D>(a, ec, t, nS, pre);
-#pragma unroll
-    for (int k = 0; k < PF; k++) {
+    auto partner = [&](int k) {
       long ep; int sl, fp;
       unpack_nbr<D, N>(nb[k], ep, sl, fp);
       psl[k] = sl;
@@ -983,8 +972,40 @@ __device__ __forceinline__ void divergence_block(const double *U, double *__rest
 #pragma unroll
         for (int v = 0; v < V; v++) pUs[k][v] = a.Utr[(ep * V + v) * nF + fp];
       }
+    };
+    auto geometry = [&](int k, int f) {
+      const double *fg = a.fgeo + ec * (D + 1) * nF + f;
+#pragma unroll
+      for (int d = 0; d < D; d++) pn[k][d] = fg[d * nF];
+      pdA[k] = fg[D * nF];
+    };
+    if constexpr (ahead) {
+      stage_U_load<D, N>(U, a, e0, neb, sr);
+#pragma unroll
+      for (int k = 0; k < PF; k++) nb[k] = a.nbr[ec * nF + (t + k * nS < nF ? t + k * nS : 0)];
+#pragma unroll
+      for (int k = 0; k < PF; k++) geometry(k, t + k * nS < nF ? t + k * nS : 0);
+      load_metric<D>(a, ec, t, nS, pij, pdet, false);
+      rk_prefetch<D>(a, ec, t, nS, pre);
+#pragma unroll
+      for (int k = 0; k < PF; k++) partner(k);
+      stage_U_store<D, N>(U, a, lops, lU, e0, neb, WU, sr);
+    } else {
+      if (valid) {
+#pragma unroll
+        for (int k = 0; k < PF; k++) {
+          const int f = t + k * nS;
+          psl[k] = 0;
+          if (f >= nF) continue;
+          nb[k] = a.nbr[ec * nF + f];
+          partner(k);
+          geometry(k, f);
+        }
+        load_metric<D>(a, ec, t, nS, pij, pdet, false);
+        rk_prefetch<D>(a, ec, t, nS, pre);
+      }
+      stage_U<D, N>(U, a, lops, lU, e0, neb, WU);
     }
-    stage_U_store<D, N>(U, a, lops, lU, e0, neb, WU, sr);
   } else {
     stage_U<D, N>(U, a, lops, lU, e0, neb, WU);
   }
