@@ -68,3 +68,12 @@ def test_euler_divergence_of_large_hexes_keeps_three_waves(kernels, N, flux):
     for self_ in (0, 1):
         k = kernels[f"k_divergence<3,{N},0,0,{flux},{self_}>"]
         assert k[".vgpr_count"] <= 168 and k[".vgpr_spill_count"] == 0, (k[".vgpr_count"], k[".vgpr_spill_count"])
+
+
+@pytest.mark.parametrize("D", [2, 3])
+def test_persistent_kernel_scratch(kernels, D):
+    """The persistent plan's kernel, a call per phase at three waves per SIMD: its scratch is
+    the call frames and a few values (236 and 532 bytes when this was written), which idle
+    threads' prologues do not add to."""
+    k = kernels[f"k_persist<{D}>"]
+    assert k[".private_segment_fixed_size"] <= (240, 540)[D - 2], k[".private_segment_fixed_size"]

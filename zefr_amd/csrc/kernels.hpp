@@ -924,7 +924,11 @@ __global__ __launch_bounds__((Shape<D, N>::kThreads)) void k_gradient(const doub
 // Euler residual is this one launch; otherwise they are read from Utr.
 // U is not __restrict__: with a fused RK update (a.rk.mode != 0) the epilogue writes a.rk.U,
 // which is the same array; U is then read only while staging, before the first barrier.
-template <int D, int N, bool VISC, int BM, int FC, bool SELF>
+// IDLE: launches of kMaxThreads threads whose tile may fill fewer (mixed multi-case launches,
+// persistent plans).  The threads beyond the tile skip the Euler prologue's loads: 16 cases of
+// 8x9 quads p=4, 50 of 256 threads in use, 7.6 us with their lines loaded and 5.8 without;
+// 16 of 3^3 hexes p=3 9.3 and 7.0.
+template <int D, int N, bool VISC, int BM, int FC, bool SELF, bool IDLE = false>
 __device__ __forceinline__ void divergence_block(const double *U, double *__restrict__ divF, const KArgs &a,
                                                  long bid) {
   using S = Shape<D, N>;
@@ -945,8 +949,9 @@ __device__ __forceinline__ void divergence_block(const double *U, double *__rest
   // barrier: first all that depends on nothing (the staged block, the partner entries and
   // face geometry of its flux points, its metric, the RK epilogue's inputs), then the partner
   // states.  Two dependent round trips; taken flux point by flux point, with the rest behind
-  // them, they were 2 FPT + 1, and on small meshes a launch is little else.  Out-of-range
-  // threads and points load a neighbour's data (in bounds) instead of branching.  (29x31x27
+  // them, they were 2 FPT + 1, and on small meshes a launch is little else.  Points beyond the
+  // last and threads of a ragged last workgroup load a neighbour's data (in bounds) instead of
+  // branching.  (29x31x27
   // hexes p=2, RK44 step 246 -> 232 us; 128^2 quads p=4, V-cycle 520 -> 495.)
   // Not so in hexes of order 6 to 8 (one element and 6 to 12 waves per workgroup, one flux
   // point at most per thread): there the lines held beside all the rest cost a wave of three
@@ -981,14 +986,16 @@ __device__ __forceinline__ void divergence_block(const double *U, double *__rest
     };
     if constexpr (ahead) {
       stage_U_load<D, N>(U, a, e0, neb, sr);
+      if (!IDLE || el < EB) {
 #pragma unroll
-      for (int k = 0; k < PF; k++) nb[k] = a.nbr[ec * nF + (t + k * nS < nF ? t + k * nS : 0)];
+        for (int k = 0; k < PF; k++) nb[k] = a.nbr[ec * nF + (t + k * nS < nF ? t + k * nS : 0)];
 #pragma unroll
-      for (int k = 0; k < PF; k++) geometry(k, t + k * nS < nF ? t + k * nS : 0);
-      load_metric<D>(a, ec, t, nS, pij, pdet, false);
-      rk_prefetch<D>(a, ec, t, nS, pre);
+        for (int k = 0; k < PF; k++) geometry(k, t + k * nS < nF ? t + k * nS : 0);
+        load_metric<D>(a, ec, t, nS, pij, pdet, false);
+        rk_prefetch<D>(a, ec, t, nS, pre);
 #pragma unroll
-      for (int k = 0; k < PF; k++) partner(k);
+        for (int k = 0; k < PF; k++) partner(k);
+      }
       stage_U_store<D, N>(U, a, lops, lU, e0, neb, WU, sr);
     } else {
       if (valid) {

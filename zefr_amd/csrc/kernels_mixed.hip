@@ -39,7 +39,7 @@ __global__ __launch_bounds__(kMaxThreads) void k_divergence_mixed(const MultiCas
   const int c = find_case(starts, nc, blockIdx.x);
   const MultiCase &m = cs[c];
   const long b = (long)blockIdx.x - starts[c];
-  ZK_SWITCH_N((divergence_block<D, N, VISC, BM, FC, !VISC>(m.U, m.out, m.a, b)))
+  ZK_SWITCH_N((divergence_block<D, N, VISC, BM, FC, !VISC, true>(m.U, m.out, m.a, b)))
 }
 
 template <int DIMS, int BM, int FC>
@@ -70,7 +70,7 @@ __global__ __launch_bounds__(kMaxThreads) void k_face_correction_mixed(const Mul
 // them inlined into one body (256 VGPRs and 76 AGPRs for the quad kernel).
 template <int D, int N, int FC, bool SELF>
 __device__ __attribute__((noinline)) void persist_div(const PersistPhase *m, long bid) {
-  divergence_block<D, N, false, 0, FC, SELF>(m->U, m->out, m->a, bid);
+  divergence_block<D, N, false, 0, FC, SELF, true>(m->U, m->out, m->a, bid);
 }
 
 template <int D, int N>
