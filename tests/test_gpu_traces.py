@@ -42,3 +42,25 @@ def test_traced_gradient_flux_only_reads_the_trace(D, order, first, beta, flux):
             out.append((dF, b.Ftr.clone()))
         assert torch.isfinite(out[0][0]).all() and out[0][1].abs().sum() > 0
         assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
+
+
+@pytest.mark.parametrize("order", [5, 6, 7, 8])
+@pytest.mark.parametrize("viscous,beta,flux", [(False, 0.5, "Rusanov"), (True, 0.5, "Roe"), (True, -0.5, "Rusanov"),
+                                               (True, 0.2, "Rusanov")])
+def test_fused_steps_of_large_hexes(order, viscous, beta, flux):
+    """Steps whose stages hand traces on (hexes of order 6 to 8) or form them from the stage
+    states (order 5): U, U_ini and every stage's residual equal the plain sequence's."""
+    import numpy as np
+    from common import TWO_PI, paired
+    n, z = (2, 3, 2), []
+    for fuse in (False, True):
+        s, _, _ = paired(dict(name=f"hand_p{order}_{viscous}_{beta}_{flux}", n=n, lo=(0.0,) * 3, hi=(TWO_PI,) * 3,
+                              order=order, viscous=viscous, state="smooth", extra={"ldg_b": beta, "fconv_type": flux}))
+        s.set_step_mode(fuse, False)
+        for _ in range(3):
+            s.do_step()
+        z.append(s)
+    np.testing.assert_array_equal(z[1].state("U"), z[0].state("U"))
+    np.testing.assert_array_equal(z[1].state("U_ini"), z[0].state("U_ini"))
+    for stage in range(4):
+        np.testing.assert_array_equal(z[1].state("divF", stage), z[0].state("divF", stage))

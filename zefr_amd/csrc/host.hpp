@@ -108,7 +108,9 @@ class Elements {
   std::vector<double> metric;                        // [E][D*D+1][nS]: adjugate(d1,d2), detJ
   // device data (element-major)
   DevBuf U_spts_d, U_ini_d, divF_d, dU_spts_d, metric_d, fgeo_d, nbr_d, ops_d, Utr_d, Gtr_d, Ftr_d;
-  DevBuf U_stage_d;  // Euler, several stages: the stage states of a fused step alternate between this and U_ini_d
+  // Euler, several stages: the stage states of a fused step alternate between this and U_ini_d
+  // (hexes of order 6 to 8: its traces, between this and Utr_d)
+  DevBuf U_stage_d;
   std::vector<double> U_host, dU_host;  // host mirrors for get_u_spts / get_du_spts
   int tile = 0;                         // elements per workgroup (0 = kernel default)
 
@@ -231,6 +233,8 @@ class FRSolver {
   // The state the residual phases read, when not U_spts_d (stages 1.. of a fused step,
   // whose stage states live in U_ini_d and U_stage_d; see step_RK_eager)
   const double *state_in = nullptr;
+  // The traces the residual phases read, when the previous stage's update wrote them
+  double *trace_in = nullptr;
   // PyFR-format solution files (src/solver.cpp:4275-4837): write returns the file name
   std::string write_solution_pyfr(const std::string &prefix);
   void restart_pyfr(const std::string &restart_case, unsigned restart_iter);
@@ -239,7 +243,8 @@ class FRSolver {
  private:
   void rk_stage_update(int stage);
   void rk_final_update();
-  void finish_with_rk(int stage, double *stage_out, bool split);
+  void finish_with_rk(int stage, double *stage_out, double *trace_out, bool split);
+  bool hands_traces() const;
   const double *cur_state() const;
   void step_RK_eager();
   void drop_graph();

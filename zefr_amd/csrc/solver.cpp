@@ -386,7 +386,8 @@ void FRSolver::viscous_flux(const zfr_ele_desc_t &d, const double *U, double *di
     auto g = d;
     g.Ftr = g.Gtr;
     status_or_throw(zfr_both_sides_flux(&g, U, divF, st));
-  } else status_or_throw(zfr_gradient_flux(&d, U, divF, st));
+  } else if (trace_in) status_or_throw(zfr_gradient_flux_traced(&d, U, divF, st));
+  else status_or_throw(zfr_gradient_flux(&d, U, divF, st));
 }
 
 // The last launch of a residual, with an epilogue or without.
@@ -480,8 +481,9 @@ void FRSolver::rk_final_update() {
 // compute_residual_finish with the RK update of this stage done by the same kernel.
 // split: the step keeps its starting state in U_spts_d until the final combination and
 // writes this stage's state to stage_out (see step_RK_eager).
-void FRSolver::finish_with_rk(int stage, double *stage_out, bool split) {
-  const auto d = eles->desc(*input, 2);
+void FRSolver::finish_with_rk(int stage, double *stage_out, double *trace_out, bool split) {
+  auto d = eles->desc(*input, 2);
+  if (trace_in) d.Utr = trace_in;
   const int ns = (int)input->nStages;
   const size_t st = eles->state_size();
   double *const A = eles->U_spts_d.as<double>(), *const I = eles->U_ini_d.as<double>();
@@ -498,6 +500,7 @@ void FRSolver::finish_with_rk(int stage, double *stage_out, bool split) {
   if (stage < ns - 1) {
     r.mode = 1;
     r.alpha = kRkAlpha[stage];
+    r.trace_out = trace_out;
   } else {
     r.mode = 2;
     for (int s = 0; s < ns; s++) r.beta[s] = (ns > 1) ? kRkBeta[s] : 1.0;
@@ -515,6 +518,19 @@ void FRSolver::finish_with_rk(int stage, double *stage_out, bool split) {
   last_launch(d, cur_state(), divF, &r, stream);
 }
 
+// Whether a fused step's stage updates also write the new state's traces for the next stage
+// to read: hexes of order 6 to 8 (one element per workgroup; a partner's line, 7 to 9 values
+// gathered for fewer flux points than the element has points, costs a stage more than a trace
+// written and read), but for Navier-Stokes at order 7, whose lines along x are whole cache
+// lines.  RK44 step, without / with traces, us per step: Euler with Rusanov 3^3 hexes p=8 62.4
+// / 56.7, 15x13x14 856 / 826, 19x17x18 p=6 813 / 747, 3^3 p=7 53.9 / 52.0, 17x15x16 p=7 999 / 985;
+// Navier-Stokes 3^3 p=8 119 / 112, 15x13x14 1514 / 1475, 19x17x18 p=6 1694 / 1559 (with Roe
+// 1715 / 1778, 4x3x4 80.6 / 77.9), 17x15x16 p=7 1517 / 1545.
+bool FRSolver::hands_traces() const {
+  if (eles->nSpts <= 256) return false;
+  return input->viscous ? onesided() && eles->order != 7 : eles->U_stage_d.p != nullptr;
+}
+
 // One RK step.  Unfused: U_ini = U, then per stage a residual and an update kernel.
 // Fused with several stages (split): the starting state stays in U_spts_d, the stage states
 // live in other buffers, and the final combination writes U_spts_d and stores the starting
@@ -527,7 +543,9 @@ void FRSolver::finish_with_rk(int stage, double *stage_out, bool split) {
 // its partners' traces from their states.  When a stage's update also wrote the new state's
 // trace for the next one to read, these bandwidth-bound kernels moved more (Euler hexes
 // p=2: 12.7 KB per element and stage, 4.3 of them traces, at 5.1 TB/s) and gained two
-// barriers.  RK44 step, with traces against without: 29x31x27 hexes p=2 Euler 238 / 191 us,
+// barriers.  Where traces are handed on all the same (hands_traces), the viscous stages write
+// them to Utr_d, which the face correction does not read; Euler stages update U_ini_d in place
+// and alternate two trace buffers, Utr_d and U_stage_d (nFpts <= nSpts there).  RK44 step, with traces against without: 29x31x27 hexes p=2 Euler 238 / 191 us,
 // Navier-Stokes 442 / 390; 32^3 hexes p=3 Euler 706 / 643, Navier-Stokes with Roe 1027 /
 // 984; 256^2 quads p=3 Euler 200 / 178; 128^2 quads p=4 Navier-Stokes 172 / 164;
 // 13x11x17 hexes p=5 Euler 163 / 157; V-cycle of 128^2 quads p=4 513 / 468.
@@ -540,26 +558,35 @@ void FRSolver::step_RK_eager() {
   if (rk_save && !split)
     hip_or_throw(hipMemcpyAsync(rk_save, eles->U_spts_d.p, eles->U_spts_d.bytes, hipMemcpyDeviceToDevice, stream),
                  "hipMemcpyAsync");
-  const bool two = split && !input->viscous && eles->U_stage_d.p;  // no second buffer: `viscous` was cleared after setup
+  const bool chain = split && hands_traces();
+  const bool two = split && !chain && !input->viscous && eles->U_stage_d.p;  // no second buffer: `viscous` was cleared after setup
   auto stage_buf = [&](int stage) {
     return (two && (ns - 2 - stage) % 2 == 0) ? eles->U_stage_d.as<double>() : eles->U_ini_d.as<double>();
+  };
+  auto trace_buf = [&](int stage) {
+    return (!input->viscous && stage % 2) ? eles->U_stage_d.as<double>() : eles->Utr_d.as<double>();
   };
   for (int stage = 0; stage < ns; stage++) {
     if (fuse_rk) {
       state_in = (split && stage > 0) ? stage_buf(stage - 1) : nullptr;
+      trace_in = (chain && stage > 0) ? trace_buf(stage) : nullptr;
       try {
         // an Euler divergence that writes the state it reads takes its partners' traces
-        if (!input->viscous && !two && (!split || stage > 0)) {
+        if (!input->viscous && !two && !trace_in && (!split || stage > 0)) {
           const auto d0 = eles->desc(*input, 0);
           status_or_throw(zfr_extrapolate(&d0, cur_state(), stream));
         }
         compute_residual_mid(stage);
-        finish_with_rk(stage, (split && stage < ns - 1) ? stage_buf(stage) : nullptr, split);
+        const bool update = split && stage < ns - 1;
+        finish_with_rk(stage, update ? stage_buf(stage) : nullptr, update && chain ? trace_buf(stage + 1) : nullptr,
+                       split);
       } catch (...) {
         state_in = nullptr;
+        trace_in = nullptr;
         throw;
       }
       state_in = nullptr;
+      trace_in = nullptr;
     } else {
       compute_residual(stage);
       if (stage < ns - 1) rk_stage_update(stage);
