@@ -77,3 +77,10 @@ def test_persistent_kernel_scratch(kernels, D):
     threads' prologues do not add to."""
     k = kernels[f"k_persist<{D}>"]
     assert k[".private_segment_fixed_size"] <= (240, 540)[D - 2], k[".private_segment_fixed_size"]
+
+
+@pytest.mark.parametrize("N", range(1, 9))
+def test_euler_roe_adjoint_of_quads_keeps_three_waves(kernels, N):
+    for form in ("k_adj_main", "k_adj_main_w64"):
+        k = kernels[f"{form}<2,{N},0,0,1>"]
+        assert k[".vgpr_count"] <= 168 and k[".vgpr_spill_count"] == 0, (k[".vgpr_count"], k[".vgpr_spill_count"])

@@ -487,8 +487,11 @@ __device__ __forceinline__ void adj_euler_block(const double *__restrict__ U, co
   const unsigned mask = valid ? owned_faces<D, N>(a.nbr + e * nF, 0) : 0u;
   const unsigned owned = face_list<D>(mask);
   const int cnt = __popc(mask) * S::nFF;
+  // quads with Roe: the metric is loaded after the face adjoint, which with it held takes 178
+  // registers instead of 168 and so two waves per SIMD instead of three
+  constexpr bool kLate = FC == 1 && D == 2;
   double ij[D][D], detJ;
-  if (valid) load_metric<D>(a, e, t, nS, ij, detJ, false);
+  if (!kLate && valid) load_metric<D>(a, e, t, nS, ij, detJ, false);
   double cp[V];
   if (t < cnt) owned_partner_trace<D, N>(U, a, e, list_fpt<D, N>(owned, t), cp);
   stage_U_store<D, N>(U, a, lops, lU, e0, neb, L::U, sr);
@@ -529,6 +532,10 @@ __device__ __forceinline__ void adj_euler_block(const double *__restrict__ U, co
       }
     }
     // volume adjoint: Dss^T w along the lines, the flux reversed
+    if (kLate) {
+      asm volatile("" ::: "memory");
+      load_metric<D>(a, e, t, nS, ij, detJ, false);
+    }
     double Us[V];
 #pragma unroll
     for (int v = 0; v < V; v++) {
@@ -572,9 +579,11 @@ __device__ __forceinline__ void adj_main_block(const double *__restrict__ U, con
 // fit it with at most a few spills, else two (256 VGPRs): held to three, 26^3 hexes p = 2
 // Euler with Roe took 129 us instead of 80 (58 spills), 100^2 quads p = 2 with Rusanov + LDG
 // 29 us instead of 25 (42 spills), while 20^2 x 27 hexes p = 3 Euler went from 80 to 76.
+// Euler quads with Roe, two / three waves, VJP: 117x102 of p=4 34.7 / 31.2 us, 185x161 of p=2
+// 34.9 / 32.7.
 template <int D, int N, bool VISC, int FC>
 struct AdjWaves {
-  static constexpr int value = FC == 0 && (!VISC || (D == 2 && (N == 4 || N == 5))) ? 3 : 2;
+  static constexpr int value = VISC ? (FC == 0 && D == 2 && (N == 4 || N == 5) ? 3 : 2) : (FC == 0 || D == 2 ? 3 : 2);
 };
 
 template <int D, int N, bool VISC, int BM, int FC>
