@@ -1701,7 +1701,14 @@ inline size_t max_lds_n(int D, int N) {
 //   nS = 64: 48^3 hexes viscous 545 against 669 (256 threads), Euler 455 against 557.
 inline int default_tile(int nS, bool phased, long nEles) {
   const int one = 64 / nS;
-  if (phased && one * nS * 32 >= 64 * 27) return one;
+  if (phased && one * nS * 32 >= 64 * 27) {
+    // elements of one point: 64 of them to a wave leave a mesh of a few ten thousand on part of
+    // the SIMDs; rather >= 1024 workgroups, of 32 elements or more (33x29x31 hexes, the
+    // one-sided kernel with 64 / 30 / 16 per workgroup: Rusanov 17.9 / 16.8 / 17.0 us, Roe 19.2 /
+    // 17.8 / 20.5; Euler residual of 31^3 8.9 with 64, 9.0 with 32, 10.8 with 16)
+    const long wgs = (nEles + 1023) / 1024;
+    return (nS == 1 && wgs < one) ? (int)(wgs < 32 ? 32 : wgs) : one;
+  }
   int best = one < 1 ? 1 : one, waves = (best * nS + 63) / 64;
   for (int w = waves + 1; w <= kMaxThreads / 64; w++) {
     const int eb = 64 * w / nS;
