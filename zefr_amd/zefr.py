@@ -269,6 +269,14 @@ class Zefr:
                 return False
         return len(s) == 3
 
+    def _refused(self, *ts):
+        """The error of a native call that failed: ValueError for a tensor it should not have
+        been given, else the library's own message."""
+        err = last_error()
+        for t in ts:
+            self._tensor_ok(t)
+        raise RuntimeError(err)
+
     # Both run on torch's current stream (torch and the library share one HIP runtime, see
     # _lib._init_torch_first), ordered with the surrounding torch work, after waiting for the
     # solver's own stream, which is non-blocking and shares the scratch.
@@ -282,8 +290,7 @@ class Zefr:
             s = U.shape
             rc = lib().zefr_residual_tensor(self._h, U.data_ptr(), out.data_ptr(), s[0], s[1], s[2],
                                             current_stream())
-            if rc == 0:
-                return out
+            return out if rc == 0 else self._refused(U, out)
         self._tensor_ok(U)
         self._tensor_ok(out)
         self.synchronize()
@@ -300,8 +307,7 @@ class Zefr:
             s = U.shape
             rc = lib().zefr_residual_vjp_tensor(self._h, U.data_ptr(), w.data_ptr(), out.data_ptr(), s[0], s[1],
                                                 s[2], current_stream())
-            if rc == 0:
-                return out
+            return out if rc == 0 else self._refused(U, w, out)
         self._tensor_ok(U)
         self._tensor_ok(w)
         self._tensor_ok(out)
