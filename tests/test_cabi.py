@@ -222,3 +222,18 @@ def test_rk_source_out_rules():
     a = _RkArgs(U=buf, U_ini=buf, divF0=buf, mode=1, stage=7, nStages=4, source=buf, source_out=buf)
     assert L.zfr_divergence_rk(C.byref(d), buf, buf, C.byref(a), None) != 0
     assert "stage out of range" in _lib.last_error(), _lib.last_error()
+
+
+@pytest.mark.parametrize("beta", [0.5, -0.5, 0.2])
+def test_viscous_divergence_needs_the_gradient_trace(beta):
+    """Whichever side's gradient enters a common flux, it is the partner's at some points of
+    every element, so a viscous divergence without Gtr is refused before any HIP call."""
+    L = _lib.lib()
+    buf = C.c_void_p(0x1000)  # never dereferenced
+    d = _lib.EleDesc(nDims=3, order=3, nVars=5, nEles=8, nSpts=64, nFpts=96, viscous=1, ldg_b=beta,
+                     gamma=1.4, prandtl=0.72, mu=1e-3, fix_vis=1, ldg_tau=0.1,
+                     ops1d=buf, metric=buf, fgeo=buf, nbr=buf, Utr=buf, Ftr=buf)
+    a = _RkArgs(U=buf, U_ini=buf, mode=1, nStages=4, alpha=0.5, dt=1e-3)
+    for rc in (L.zfr_divergence(C.byref(d), buf, buf, None),
+               L.zfr_divergence_rk(C.byref(d), buf, buf, C.byref(a), None)):
+        assert rc != 0 and "Gtr is NULL" in _lib.last_error(), _lib.last_error()

@@ -383,7 +383,7 @@ int zfr_divergence(const zfr_ele_desc_t *d, const double *U, double *divF, void 
   if (!rc) rc = need_arg(U, "U");
   if (!rc) rc = need_arg(divF, "divF");
   if (!rc && d->viscous) rc = need(d->Utr, "Utr");
-  if (!rc && d->viscous && d->ldg_b != 0.5 && d->ldg_b != -0.5) rc = need(d->Gtr, "Gtr");
+  if (!rc && d->viscous) rc = need(d->Gtr, "Gtr");
   if (rc) return rc;
   return zk::dispatch(zk::Op::Div, d, U, divF, (hipStream_t)stream);
 }
@@ -495,7 +495,7 @@ int rk_fused(zk::Op op, const zfr_ele_desc_t *d, const double *U, double *divF, 
   const bool reads_tr = op == zk::Op::Div && (d->viscous || zk::rk_writes_input(rk, U));
   int rc = need_geometry(d);
   if (!rc && reads_tr) rc = need(d->Utr, "Utr");
-  if (!rc && op == zk::Op::Div && d->viscous && d->ldg_b != 0.5 && d->ldg_b != -0.5) rc = need(d->Gtr, "Gtr");
+  if (!rc && op == zk::Op::Div && d->viscous) rc = need(d->Gtr, "Gtr");
   if (!rc && (op == zk::Op::FaceCorr || op == zk::Op::FaceCorrBoth)) rc = need(d->Ftr, "Ftr");
   if (rc) return rc;
   if (update && (r->nStages < 1 || r->nStages > zk::kMaxRkStages || r->stage < 0 || r->stage >= r->nStages))
