@@ -64,3 +64,65 @@ def test_fused_steps_of_large_hexes(order, viscous, beta, flux):
     np.testing.assert_array_equal(z[1].state("U_ini"), z[0].state("U_ini"))
     for stage in range(4):
         np.testing.assert_array_equal(z[1].state("divF", stage), z[0].state("divF", stage))
+
+
+SHAPES = [(2, 0, 2), (2, 1, 3), (2, 4, 3), (2, 5, 2), (3, 1, 4), (3, 2, 3), (3, 3, 5), (3, 6, 3)]
+
+
+def _stage(b, dF, X, tr):
+    from test_cabi import _RkArgs
+    return _RkArgs(U=ptr(X), U_ini=ptr(b.U), divF0=ptr(dF), mode=1, stage=0, nStages=4, alpha=0.5, dt=1e-3,
+                   trace_out=ptr(tr))
+
+
+@pytest.mark.parametrize("D,order,first", SHAPES)
+@pytest.mark.parametrize("beta", [0.5, -0.5])
+def test_face_correction_writes_the_next_trace(D, order, first, beta):
+    """zfr_face_correction_rk with trace_out: the partner-owned half of the new state's trace,
+    as zfr_extrapolate_partner writes it, the other points untouched; the next launch reads it."""
+    import torch
+    L, b = _lib.lib(), Block(D, order, first=first)
+    owner = 0 if beta == 0.5 else 1
+    for tile in (0, 1, 3, 4):
+        d, dF, X = b.desc(beta=beta, tile=tile), b.field(), b.field()
+        b.Utr.fill_(7.0)
+        want, tr = b.Utr.clone(), b.Utr.clone()
+        torch.cuda.synchronize()
+        ok(L.zfr_gradient_flux(C.byref(d), ptr(b.U), ptr(dF), None))
+        ok(L.zfr_face_correction_rk(C.byref(d), ptr(dF), C.byref(_stage(b, dF, X, tr)), None))
+        d.Utr = ptr(want)
+        ok(L.zfr_extrapolate_partner(C.byref(d), ptr(X), None))
+        torch.cuda.synchronize()
+        assert torch.isfinite(X).all() and not torch.equal(X, b.U)
+        assert torch.equal(tr, want)
+        assert torch.equal((tr == 7.0).all(1), b.slot == owner)
+        R = [b.field(), b.field()]
+        torch.cuda.synchronize()
+        d.Utr = ptr(tr)
+        ok(L.zfr_gradient_flux_traced(C.byref(d), ptr(X), ptr(R[0]), None))
+        ok(L.zfr_face_correction(C.byref(d), ptr(R[0]), None))
+        d.Utr = ptr(b.Utr)
+        ok(L.zfr_gradient_flux(C.byref(d), ptr(X), ptr(R[1]), None))
+        ok(L.zfr_face_correction(C.byref(d), ptr(R[1]), None))
+        torch.cuda.synchronize()
+        assert torch.equal(R[0], R[1])
+
+
+@pytest.mark.parametrize("D,order,first", SHAPES)
+@pytest.mark.parametrize("beta", [0.2, 0.0])
+def test_both_sides_correction_writes_the_next_trace(D, order, first, beta):
+    """zfr_both_sides_correction with trace_out: the whole trace, as zfr_extrapolate writes it
+    (which zfr_gradient and zfr_divergence read)."""
+    import torch
+    L, b = _lib.lib(), Block(D, order, first=first)
+    for tile in (0, 1, 3, 4):
+        d, dF, X = b.desc(beta=beta, tile=tile), b.field(), b.field()
+        tr = torch.full_like(b.Utr, 7.0)
+        b.Utr.fill_(7.0)
+        torch.cuda.synchronize()
+        ok(L.zfr_both_sides_flux(C.byref(d), ptr(b.U), ptr(dF), None))
+        ok(L.zfr_both_sides_correction(C.byref(d), ptr(dF), C.byref(_stage(b, dF, X, tr)), None))
+        ok(L.zfr_extrapolate(C.byref(d), ptr(X), None))
+        torch.cuda.synchronize()
+        assert torch.isfinite(X).all() and not torch.equal(X, b.U)
+        assert torch.equal(tr, b.Utr)
