@@ -178,7 +178,6 @@ void launch_multi(const MultiGroup &g, hipStream_t st) {
   const long *s0 = g.starts;
   switch (g.op) {
     case Op::Extrap:
-    case Op::ExtrapPartner:
       hipLaunchKernelGGL((k_extrapolate_multi<D, N>), grid, block, g.lds, st, c, s0, g.nc);
       break;
     case Op::Div:  // Euler
