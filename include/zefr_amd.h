@@ -187,8 +187,9 @@ int zefr_set_step_mode(zefr_t *z, int fuse_rk, int use_graph);
  * with the reason.  Results are identical to the eager and graph cycles. */
 int zefr_set_pmg_persistent(zefr_t *z, int on);
 /* Run `reps` residuals (stage 0) with HIP events around each kernel on the solver's
- * stream; ms_out[0..2] = average duration of the extrapolate / gradient / divergence
- * launch (gradient is 0 for inviscid runs).  No counterpart in the reference: this is the
+ * stream; ms_out[0..2] = average duration of the trace launch (none: the gap between two
+ * events), of the first viscous launch (the same gap for inviscid runs) and of the last
+ * launch (face correction, or the Euler divergence).  No counterpart in the reference: this is the
  * timing hook of the benchmark. */
 int zefr_time_residual_kernels(zefr_t *z, int reps, double *ms_out);
 /* divF = R(U) for an arbitrary device state U (device layout [E][V][nS], as
@@ -200,7 +201,7 @@ int zefr_time_residual_kernels(zefr_t *z, int reps, double *ms_out);
 int zefr_residual_at(zefr_t *z, const double *U, double *divF, void *stream);
 /* v = (dR/dU)^T w at U (all device pointers, layout [E][V][nS]) on `stream` (NULL: the
  * null stream): the residual's vector-Jacobian product (new; no reference counterpart).
- * Euler, or Navier-Stokes with LDG beta = +-1/2.  Same scratch rule as residual_at. */
+ * Same scratch rule as residual_at; v may be w, and must not overlap U. */
 int zefr_residual_vjp(zefr_t *z, const double *U, const double *w, double *v, void *stream);
 /* The same on arrays of a stated shape, which must be the solver's [nEles][nVars][nSpts]; they
  * wait for the solver's own stream (on the host) before they launch on `stream`. */
@@ -407,7 +408,8 @@ int zfr_face_correction_rk(const zfr_ele_desc_t *d, double *divF, const zfr_rk_a
  * in each common flux, src/faces.cpp:1476-1614), as zfr_gradient_flux and zfr_face_correction
  * are for beta = +-1/2: the first writes the volume part of divF and this side's share of the
  * common flux at every flux point to d->Ftr, the second adds both sides' shares.  rk: an
- * epilogue as in zfr_face_correction_rk (trace_out takes every flux point), or NULL. */
+ * epilogue as in zfr_face_correction_rk, or NULL (trace_out takes every flux point, as
+ * zfr_extrapolate writes them; zfr_gradient and zfr_divergence read such a trace). */
 int zfr_both_sides_flux(const zfr_ele_desc_t *d, const double *U, double *divF, void *stream);
 int zfr_both_sides_correction(const zfr_ele_desc_t *d, double *divF, const zfr_rk_args_t *rk, void *stream);
 int zfr_divergence_rk(const zfr_ele_desc_t *d, const double *U, double *divF, const zfr_rk_args_t *rk,

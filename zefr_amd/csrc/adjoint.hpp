@@ -593,8 +593,8 @@ void k_adj_main(const double *__restrict__ U, const double *__restrict__ w, doub
   adj_main_block<D, N, VISC, BM, FC>(U, w, Wtr, Xtr, vout, a, xcd_block(blockIdx.x, gridDim.x));
 }
 
-// The same kernel for workgroups of one wave (the viscous adjoint runs one element per
-// workgroup; one wave for hex p=3): its barriers need no cross-wave synchronisation.
+// The same kernel for workgroups of one wave (the default tile where a wave is well filled, see
+// default_tile): its barriers need no cross-wave synchronisation.
 template <int D, int N, bool VISC, int BM, int FC>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(AdjWaves<D, N, VISC, FC>::value)))
 void k_adj_main_w64(const double *__restrict__ U, const double *__restrict__ w, double *__restrict__ Wtr,

@@ -14,21 +14,25 @@
 //    integer map (no pointer tables), and computes the common solution / common flux for
 //    its own side of the face.  Both sides evaluate the same formula on the same L/R
 //    states, so the interface flux stays single-valued.
-//  * Navier-Stokes with a general LDG beta needs two grid-wide dependencies (U traces,
-//    then gradient traces), so a residual is three launches: extrapolate -> gradient ->
-//    divergence.  The divergence kernel recomputes the corrected gradient instead of
-//    storing it: re-reading U and the U trace costs less HBM traffic than writing and
-//    re-reading the gradient.
 //  * With LDG beta = +-1/2 (the usual setting) only one side's gradient enters each
 //    common flux and the common solution is the other side's trace, so the "owner" side
 //    can finish the whole common flux right after its own gradient, and the only other-
 //    side data it needs (the partner's trace at its owned points) it extrapolates from the
 //    partner's U itself: gradient_flux (gradient, volume divergence, owned common fluxes)
 //    -> face_correction, two launches.  No gradient trace is stored at all.
-//  * Euler: divergence alone, extrapolating the partner traces from the partner's U (with
-//    a fused RK update: extrapolate -> divergence, since the update overwrites U).
+//  * Navier-Stokes with a general LDG beta runs through the same two kernels: each side writes
+//    its weighted share of the common flux (both_sides_flux -> both_sides_correction).  The
+//    three launches with gradient traces (extrapolate -> gradient -> divergence, whose last
+//    one alone writes, and only its own elements) serve a residual over its own state.
+//  * Euler: divergence alone, extrapolating the partner traces from the partner's U; a fused
+//    RK update writes another buffer, or in place reads the traces that a launch or the update
+//    before it wrote.
 //
-// All arithmetic is FP64.  Reference call sites are cited at each kernel.
+// All arithmetic is FP64.  Reference call sites are cited at each kernel.  Times in the
+// comments: microseconds per residual, VJP, step or V-cycle by the host clock over 20 calls or
+// more between two waits, the smallest of several such bursts, both forms in turn on one card;
+// where a kernel is named alone, its mean in rocprofv3's trace.  Longer runs at steady clocks
+// give smaller figures (V-cycle of 128^2 quads p=4: 450 in bursts, 335 in long runs).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -1255,11 +1259,13 @@ __global__ __launch_bounds__((Shape<D, N>::kThreads)) void k_divergence_multi(co
 // gradient and both sides' fluxes formed again) took 84 us per residual of 21x23x19 hexes
 // p=2 and 1.94 ms of 48^2 x 49 hexes p=3.
 
-// Register budget: three waves per SIMD for hex p=3 and 4.  At p=3 the kernel's LDS admits 15 waves per CU,
-// but 3.2 per SIMD are in flight on average, with the LDS pipe 70% and the VALU 54% busy
-// (64^3, rocprofv3), so a fourth wave buys nothing: held to 128 VGPRs the Roe kernel spills
-// 10 of them (0.37 GB written and read back per residual; 64^3 residual 1627 us), at 148 it
-// spills none (1488 us).  Rusanov takes 124 either way.  Other shapes keep the default
+// Register budget: three waves per SIMD for hex p=3 and 4.  At p=3 the kernel's LDS admits 15
+// waves per CU, but 3.2 per SIMD are in flight on average, with the LDS pipe 70% and the VALU
+// 54% busy (64^3, rocprofv3), so a fourth wave buys nothing: held to 128 VGPRs the Roe kernel
+// spills 10 of them (0.37 GB written and read back per residual; 64^3 residual 1627 us), at
+// 148 it spills none (1488 us).  Rusanov takes 124 either way.  At p=4 beta = +-1/2 takes 144
+// by itself; a general beta would take 175, two waves, and at three spills 6 to 10 (14x12x13,
+// two / three waves: Rusanov 52.0 / 49.2 us, Roe 52.6 / 49.8).  Other shapes keep the default
 // allocation.
 template <int D, int N>
 struct OneSidedWaves {
@@ -1299,7 +1305,10 @@ __device__ __forceinline__ void visc_onesided_block(const double *__restrict__ U
   // element's lanes, nS apart: hexes have 3 / N of the lanes busy and lose as much by the second
   // element index (64^3 p=3 Roe 1530 / 1580 us, 13x11x17 p=5 71 / 77), quads p=3 gain nothing
   // (256^2 67 / 70).  In lanes / in a row: 256^2 quads p=4 112 / 105 us, with Roe 115 / 112;
-  // 96x100 23.0 / 21.8; 200x201 p=5 106 / 97; 150x151 p=6 90 / 80; 24^2 p=6 11.7 / 11.7.
+  // 96x100 23.0 / 21.8; 200x201 p=5 106 / 97; 150x151 p=6 90 / 80; 24^2 p=6 11.7 / 11.7.  Not
+  // where an element fills waves of its own (nS a multiple of 64: quads p=7), whose default
+  // tile is one element, so that a row is its own lanes again (73x64 p=7 30.4 / 31.2, with Roe
+  // 30.8 / 32.0).
   // A thread takes its item in the prologue and again in the face phase, so with SELF the
   // partner's trace there stays in its registers (a second item, nS further, is rare for
   // N >= 3; its trace is parked in Utr at the element's own point, which nothing else reads).
@@ -1492,8 +1501,8 @@ __device__ __forceinline__ void visc_onesided_block(const double *__restrict__ U
         }
       }
       asm volatile("" ::: "memory");
-      // one variable's line at a time (a compiler barrier after each): 128 VGPRs instead of
-      // 160, i.e. one more wave per SIMD, worth more than the loads' overlap
+      // one variable's line at a time (a compiler barrier after each): all lines in flight at
+      // once take some 30 VGPRs more, spilled or a wave less in the shapes that are full
       visc_normal<D>(Uo, [&](int j, double *dUj) {
 #pragma unroll
         for (int v = 0; v < V; v++) {
@@ -1699,6 +1708,12 @@ inline size_t max_lds_n(int D, int N) {
 //   nS = 49, filled to 49/64: viscous 192^2 quads 121 against 107, Euler 68 against 60;
 //   nS = 27, filled to 27/32: 40^3 hexes viscous 185 against 194, Euler 113 against 136;
 //   nS = 64: 48^3 hexes viscous 545 against 669 (256 threads), Euler 455 against 557.
+// The main adjoint kernels alone, one wave against the best-filled tile (3e5 points):
+//   nS = 25: quads p=4 Rusanov 34.4 against 31.1, Euler 18.9 / 17.7, general beta 26.6 / 24.7;
+//   nS = 27: hexes p=2 Rusanov 68 against 78, Roe 76 / 86, Euler 27 / 27, general beta 47 / 50;
+//   nS = 16: quads p=3 27.0 against 29.4, 32.5 / 35.5, 15.0 / 15.7, 21.6 / 23.7;
+//   nS = 64: hexes p=3 61 against 78, 69 / 93, 22.2 / 23.3, 46 / 51
+// (k_adj_main_gen has no one-wave form: its fewer waves wait less for one another).
 inline int default_tile(int nS, bool phased, long nEles) {
   const int one = 64 / nS;
   if (phased && one * nS * 32 >= 64 * 27) {
@@ -1771,8 +1786,7 @@ struct AdjPtrs {
   const KArgs::Rk *rk = nullptr;  // fused RK update for Div / FaceCorr
 };
 
-// LDS doubles per element of each kernel (the owned-point list of the one-sided kernel is
-// nF + 1 ints).
+// LDS doubles per element of each kernel.
 template <int D, int N>
 size_t lds_per_element(Op op, bool viscous) {
   using S = Shape<D, N>;

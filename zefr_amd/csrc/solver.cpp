@@ -612,7 +612,7 @@ void FRSolver::set_step_mode(bool fuse, bool use) {
 }
 
 // step_RK (src/solver.cpp:2865-3097) with a supplied dt.  With use_graph the step's
-// launches (the U_ini copy, three kernels per stage) are captured once and replayed; the
+// launches (fused: one per Euler stage, two per viscous one) are captured once and replayed; the
 // kernel arguments bake in dt and the tile, so a change of either recaptures.
 void FRSolver::step_RK() {
   need_device(*this);
