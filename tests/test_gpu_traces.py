@@ -49,21 +49,23 @@ def test_traced_gradient_flux_only_reads_the_trace(D, order, first, beta, flux):
                                                (True, 0.2, "Rusanov")])
 def test_fused_steps_of_large_hexes(order, viscous, beta, flux):
     """Steps whose stages hand traces on (hexes of order 6 to 8) or form them from the stage
-    states (order 5): U, U_ini and every stage's residual equal the plain sequence's."""
+    states (order 5), launched or replayed from a graph: U, U_ini and every stage's residual
+    equal the plain sequence's."""
     import numpy as np
     from common import TWO_PI, paired
     n, z = (2, 3, 2), []
-    for fuse in (False, True):
+    for fuse, graph in ((False, False), (True, False), (True, True)):
         s, _, _ = paired(dict(name=f"hand_p{order}_{viscous}_{beta}_{flux}", n=n, lo=(0.0,) * 3, hi=(TWO_PI,) * 3,
                               order=order, viscous=viscous, state="smooth", extra={"ldg_b": beta, "fconv_type": flux}))
-        s.set_step_mode(fuse, False)
+        s.set_step_mode(fuse, graph)
         for _ in range(3):
             s.do_step()
         z.append(s)
-    np.testing.assert_array_equal(z[1].state("U"), z[0].state("U"))
-    np.testing.assert_array_equal(z[1].state("U_ini"), z[0].state("U_ini"))
-    for stage in range(4):
-        np.testing.assert_array_equal(z[1].state("divF", stage), z[0].state("divF", stage))
+    for s in z[1:]:
+        np.testing.assert_array_equal(s.state("U"), z[0].state("U"))
+        np.testing.assert_array_equal(s.state("U_ini"), z[0].state("U_ini"))
+        for stage in range(4):
+            np.testing.assert_array_equal(s.state("divF", stage), z[0].state("divF", stage))
 
 
 SHAPES = [(2, 0, 2), (2, 1, 3), (2, 4, 3), (2, 5, 2), (3, 1, 4), (3, 2, 3), (3, 3, 5), (3, 6, 3)]
